@@ -53,6 +53,7 @@
 // the blocks resident on one XCD share A rows and W columns in its L2.
 #include "tb_common.h"
 #include "prefill_plan.h"
+#include "w4a16_tile.h"
 
 #include <algorithm>
 #include <functional>
@@ -65,89 +66,12 @@
 namespace tb {
 namespace w4a16 {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int BM = 256, BN = 256, BK = 64;
+constexpr int BM = 256, BN = 256;
 constexpr int GROUP_M = 4;  // tile rows per ordering group
 
 struct Tile {
   int m0, n0;
 };
-
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-constexpr uint32_t RSRC_DW3 = 0x00020000u;
-constexpr uint32_t OOB = 0x80000000u;
-__device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, (int)RSRC_DW3);
-}
-
-// Row map of the MoE pipeline's tiles: tile row m is (token, slot) pair
-// ids[m]; the pair's token is ids[m] / topk and its routing weight w[ids[m]].
-struct RowMap {
-  const int* ids = nullptr;
-  const float* w = nullptr;
-  int topk = 1;
-  int pairs = 0;
-};
-
-// fp16 of an fp32 value that is already rounded: the empty asm keeps the
-// conversion from being folded into the preceding multiply (a mixed-precision
-// FMA would round the exact product once, not the fp32 product).
-__device__ __forceinline__ _Float16 h_of_rounded(float f) {
-  asm volatile("" : "+v"(f));
-  return (_Float16)f;
-}
-
-// Expert and row range of grouped tile row mt: rows offsets[e] .. offsets[e+1]
-// of the row space (R rows) use expert e, cut into 256-row tiles.  Offsets are
-// clamped to [0, R] so that malformed ones never address rows outside A / Y.
-// Returns false past the last tile.  Every wavefront searches 64 experts at a
-// time, one per lane (a prefix sum of tile counts, then a ballot), so the
-// search costs a few loads in flight together rather than one dependent load
-// per expert.
-__device__ __forceinline__ bool grouped_tile(const int* __restrict__ offsets, int experts, int R, int mt, int& e,
-                                             int& m0, int& m_end) {
-  const int lane = threadIdx.x & 63;
-  int seen = 0;
-  for (int x0 = 0; x0 < experts; x0 += 64) {
-    const int x = x0 + lane;
-    int lo = 0, hi = 0;
-    if (x < experts) {
-      lo = min(max(offsets[x], 0), R);
-      hi = min(max(offsets[x + 1], lo), R);
-    }
-    const int cnt = (hi - lo + BM - 1) / BM;
-    int incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int o = __shfl_up(incl, d);
-      if (lane >= d) incl += o;
-    }
-    const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
-    if (mt < seen + total) {
-      const unsigned long long hit = __ballot(seen + incl > mt);
-      const int l = __builtin_ctzll(hit);
-      const int lo_l = __shfl(lo, l), hi_l = __shfl(hi, l), before = seen + __shfl(incl - cnt, l);
-      // uniform across the block: scalar registers, so that every address
-      // derived from the tile stays scalar
-      e = __builtin_amdgcn_readfirstlane(x0 + l);
-      m0 = __builtin_amdgcn_readfirstlane(lo_l + (mt - before) * BM);
-      m_end = __builtin_amdgcn_readfirstlane(hi_l);
-      return true;
-    }
-    seen += total;
-  }
-  return false;
-}
-
-__device__ __forceinline__ int grouped_block_id() {
-  const int nb = gridDim.x;
-  int bid = blockIdx.x;
-  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  return bid;
-}
 
 // ---------------------------------------------------------------------------
 // Decode kernel (M <= 16, HBM-bound on the weights).  A block of eight
@@ -462,22 +386,6 @@ constexpr size_t C_BYTES = (size_t)BM * C_STRIDE * 2;  // 132 KiB
 constexpr size_t LDS_BYTES = RING_BYTES > C_BYTES ? RING_BYTES : C_BYTES;
 static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 
-typedef int v2i __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ void dma16(uint32_t lds_addr, uint32_t voff, const i32x4& rsrc, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(rsrc),
-                 "s"(__builtin_amdgcn_readfirstlane((int)soff))
-               : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(uint32_t lds_addr, uint32_t voff, const i32x4& rsrc, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(rsrc),
-                 "s"(__builtin_amdgcn_readfirstlane((int)soff))
-               : "memory", "m0");
-}
 // Block ids go round-robin to the 8 XCDs: regroup ids so that each XCD owns
 // a contiguous run of tiles (when the count is a multiple of 8).
 __device__ __forceinline__ int remap_xcd(int bid, int nb) {
@@ -499,29 +407,6 @@ __device__ __forceinline__ Tile tile_in_grid(int idx, int tiles_m, int tiles_n, 
 __device__ __forceinline__ Tile tile_of(int bid, int nb, int tiles_m, int tiles_n, int rows, int n_base) {
   return tile_in_grid(remap_xcd(bid, nb), tiles_m, tiles_n, rows, n_base);
 }
-__device__ __forceinline__ i32x4 rsrc4(const void* p, uint32_t bytes) {
-  const uint64_t base = (uint64_t)(uintptr_t)p;
-  i32x4 r;
-  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)base);
-  r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32) & 0xFFFF);
-  r[2] = __builtin_amdgcn_readfirstlane((int)bytes);
-  r[3] = (int)RSRC_DW3;
-  return r;
-}
-// (x & mask) | c in one instruction: mask from a scalar register, c from a vector one
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t c) {
-  uint32_t r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(c));
-  return r;
-}
-
-// What a tile reads and writes besides the plain product.
-enum TileMode {
-  T_PLAIN = 0,    // rows m < M of A and Y
-  T_GATE_UP = 1,  // MoE gate/up: see below
-  T_DOWN = 2      // MoE down: see below
-};
-
 // One tile at (m0, n0): the eight wavefronts as 8 / WN row groups of 32 MB
 // rows times WN column groups of 64 columns.  WN = 4: 256 columns and 64 MB
 // rows (MB = 4: 256, MB = 3: 192); WN = 2, MB = 2: 256 rows x 128 columns,
@@ -1332,10 +1217,10 @@ __global__ void __launch_bounds__(256, 1)
 
 // Grouped (MoE) variant: rows offsets[e] .. offsets[e+1] of A use expert e's
 // weights.  The grid is an upper bound (sum over experts of ceil(rows / 256)
-// <= R / 256 + E tile rows, times the N tiles); each block walks the E + 1
-// offsets to find its expert and tile row, and blocks past the last tile exit.
-// Tile ids are regrouped per XCD as in the dense kernel, so the blocks
-// resident on one XCD work on neighbouring tiles of the same expert.  A tile
+// <= R / 256 + E tile rows, times the N tiles); each block counts the tiles
+// that exist, takes its share (grouped_tile) and finds its expert and tile
+// row, and blocks past the last tile exit.  An XCD's blocks work on
+// neighbouring tiles of the same expert.  A tile
 // is the dense kernel's 256 x 256 tile on the expert's operands, its A and Y
 // based at the tile's first row with the rows up to the expert's last as the
 // valid ones, so each expert segment equals the dense product bit for bit.
@@ -1345,10 +1230,8 @@ __global__ void __launch_bounds__(256, 1)
                   int experts, int N, int K, int group, int tiles_n) {
   extern __shared__ __attribute__((aligned(16))) _Float16 lds_h[];
   uint8_t* const lds = reinterpret_cast<uint8_t*>(lds_h);
-  const int bid = grouped_block_id();
-  const int mt = bid / tiles_n, nt = bid - mt * tiles_n;
-  int e = 0, m0 = 0, m_end = 0;
-  if (!grouped_tile(offsets, experts, R, mt, e, m0, m_end)) return;  // beyond the last tile: uniform
+  int e = 0, m0 = 0, m_end = 0, nt = 0;
+  if (!grouped_tile<BM>(offsets, experts, R, tiles_n, e, m0, m_end, nt)) return;  // beyond the last tile: uniform
   const int64_t wstride = (int64_t)K * (N / 2), sstride = (int64_t)(K / group) * N, zstride = (int64_t)(K / group) * (N / 2);
   // a last column tile of at most 128 columns (N = 1408 is 5.5 tiles) runs
   // as 256 x 128: half the MFMAs, the same dequantisation per wavefront
@@ -1372,10 +1255,8 @@ __global__ void __launch_bounds__(256, 1)
                 int tiles_n) {
   extern __shared__ __attribute__((aligned(16))) _Float16 lds_h[];
   uint8_t* const lds = reinterpret_cast<uint8_t*>(lds_h);
-  const int bid = grouped_block_id();
-  const int mt = bid / tiles_n, nt = bid - mt * tiles_n;
-  int e = 0, m0 = 0, m_end = 0;
-  if (!grouped_tile(offsets, experts, pairs, mt, e, m0, m_end)) return;
+  int e = 0, m0 = 0, m_end = 0, nt = 0;
+  if (!grouped_tile<BM>(offsets, experts, pairs, tiles_n, e, m0, m_end, nt)) return;
   const int N = 2 * I;
   const int64_t wstride = (int64_t)K * I, sstride = (int64_t)(K / group) * N, zstride = (int64_t)(K / group) * I;
   RowMap rm;
@@ -1383,10 +1264,10 @@ __global__ void __launch_bounds__(256, 1)
   rm.topk = topk;
   rm.pairs = pairs;
   if (I - nt * (BN / 2) <= BN / 4)
-    p8::tile4<4, 2, p8::T_GATE_UP>(lds, X, W + e * wstride, S + e * sstride, Z + e * zstride, act + (int64_t)m0 * I,
+    p8::tile4<4, 2, T_GATE_UP>(lds, X, W + e * wstride, S + e * sstride, Z + e * zstride, act + (int64_t)m0 * I,
                                    m_end - m0, N, K, group, Tile{0, nt * BN}, tokens, rm);
   else
-    p8::tile4<8, 4, p8::T_GATE_UP>(lds, X, W + e * wstride, S + e * sstride, Z + e * zstride, act + (int64_t)m0 * I,
+    p8::tile4<8, 4, T_GATE_UP>(lds, X, W + e * wstride, S + e * sstride, Z + e * zstride, act + (int64_t)m0 * I,
                                    m_end - m0, N, K, group, Tile{0, nt * BN}, tokens, rm);
 }
 
@@ -1400,20 +1281,18 @@ __global__ void __launch_bounds__(p8::THREADS, 1)
              int group, int tiles_n) {
   extern __shared__ __attribute__((aligned(16))) _Float16 lds_h[];
   uint8_t* const lds = reinterpret_cast<uint8_t*>(lds_h);
-  const int bid = grouped_block_id();
-  const int mt = bid / tiles_n, nt = bid - mt * tiles_n;
-  int e = 0, m0 = 0, m_end = 0;
-  if (!grouped_tile(offsets, experts, pairs, mt, e, m0, m_end)) return;
+  int e = 0, m0 = 0, m_end = 0, nt = 0;
+  if (!grouped_tile<BM>(offsets, experts, pairs, tiles_n, e, m0, m_end, nt)) return;
   const int64_t wstride = (int64_t)I * (H / 2), sstride = (int64_t)(I / group) * H, zstride = (int64_t)(I / group) * (H / 2);
   RowMap rm;
   rm.ids = ids + m0;
   rm.w = w;
   rm.pairs = pairs;
   if (H - nt * BN <= BN / 2)
-    p8::tile8<2, 2, p8::T_DOWN>(lds, act + (int64_t)m0 * I, W + e * wstride, S + e * sstride, Z + e * zstride, Y,
+    p8::tile8<2, 2, T_DOWN>(lds, act + (int64_t)m0 * I, W + e * wstride, S + e * sstride, Z + e * zstride, Y,
                                 m_end - m0, H, I, group, Tile{0, nt * BN}, m_end - m0, rm);
   else
-    p8::tile8<4, 4, p8::T_DOWN>(lds, act + (int64_t)m0 * I, W + e * wstride, S + e * sstride, Z + e * zstride, Y,
+    p8::tile8<4, 4, T_DOWN>(lds, act + (int64_t)m0 * I, W + e * wstride, S + e * sstride, Z + e * zstride, Y,
                                 m_end - m0, H, I, group, Tile{0, nt * BN}, m_end - m0, rm);
 }
 
