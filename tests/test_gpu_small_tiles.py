@@ -1,0 +1,99 @@
+"""GPU parity of the small W4A16 tiles (w4a16_small.hip): every tile of the
+grouped, gate/up and down products against the CPU oracle, and bit for bit
+against the 256-row tiles on the same rows."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from small_tile_cases import EXPERT_TILES
+from tilebench_amd import runtime as rt
+from tilebench_amd.data import tensors as T
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(*a):
+    print("[gpu case]", *a, flush=True)
+
+
+def _grouped(rows, N, K, G, seed):
+    g = T._gen(seed)
+    off = torch.zeros(len(rows) + 1, dtype=torch.int32)
+    off[1:] = torch.cumsum(torch.tensor(rows), 0)
+    A = torch.randn(int(off[-1]), K, generator=g).to(torch.float16)
+    return (A, *T.random_int4_weights(K, N, G, g, experts=len(rows)), off)
+
+
+@pytest.mark.parametrize("tile", list(EXPERT_TILES))
+def test_grouped_tiles_match_oracle(gpu, tile):
+    from tilebench_amd.benchmarks.operators.moe_w4a16_grouped_gemm import impl_hip
+
+    for rows, N, K, G in EXPERT_TILES[tile]:
+        _say("grouped", tile, sum(rows), len(rows), N, K, G)
+        A, p, s, z, off = _grouped(rows, N, K, G, seed=N + K)
+        Y = impl_hip.run(*(t.to(gpu) for t in (A, p, s, z, off)), G)
+        torch.cuda.synchronize()
+        ref = oracle.moe_w4a16_grouped_gemm(A.numpy(), p.numpy(), s.numpy(), z.numpy(), off.numpy(), G)
+        np.testing.assert_allclose(Y.cpu().numpy().astype(np.float32), ref.astype(np.float32), atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("per_expert", [1, 20, 60])  # 32 x 128 (one column), 32 x 256 and 64 x 256 tiles
+def test_grouped_rows_do_not_depend_on_the_tile(gpu, per_expert):
+    """The first rows of every expert alone give the bits they have in a call
+    whose experts fill 256-row tiles."""
+    from tilebench_amd.benchmarks.operators.moe_w4a16_grouped_gemm import impl_hip
+
+    rows, N, K, G = EXPERT_TILES["256"][0]
+    _say("grouped rows", per_expert)
+    A, p, s, z, off = _grouped(rows, N, K, G, seed=5)
+    d = [t.to(gpu) for t in (A, p, s, z)]
+    big = impl_hip.run(*d, off.to(gpu), G)
+    take = [min(r, per_expert) for r in rows]
+    o2 = torch.zeros(len(rows) + 1, dtype=torch.int32)
+    o2[1:] = torch.cumsum(torch.tensor(take), 0)
+    idx = torch.cat([torch.arange(int(off[e]), int(off[e]) + n) for e, n in enumerate(take)]).to(gpu)
+    small = impl_hip.run(d[0][idx].contiguous(), *d[1:], o2.to(gpu), G)
+    torch.cuda.synchronize()
+    assert torch.equal(small.view(torch.int16), big[idx].view(torch.int16))
+
+
+@pytest.mark.parametrize("Tk,E,k,H,I,g", [(1, 8, 4, 256, 128, 64), (33, 5, 3, 320, 72, 64), (70, 70, 2, 192, 704, 64),
+                                          (500, 16, 8, 128, 704, 64), (700, 16, 8, 192, 1032, 64)])
+def test_gate_up_and_down_tiles_match_oracle(gpu, Tk, E, k, H, I, g):
+    """Token gather, SiLU epilogue, routing weights and the scatter on each
+    tile; I % 32 != 0 and H % 32 != 0 take the 4-byte weight loads.  Pairs
+    routed nowhere stay unwritten."""
+    _say("gate_up + down", Tk, E, k, H, I, g)
+    gen = T._gen(Tk + I)
+    X = torch.randn(Tk, H, generator=gen).to(torch.float16)
+    ids = T.zipf_routing(Tk, k, E, 1.1, seed=7).to(torch.int32)
+    if Tk > 1:
+        ids[::5, 0] = E + 2
+    w = torch.rand(Tk, k, generator=gen)
+    sid, off = oracle.moe_align(ids.numpy(), E)
+    P = Tk * k
+    sorted_ids = np.full(P, -1, np.int32)
+    sorted_ids[:len(sid)] = sid
+    dev = {n: t.to(gpu) for n, t in dict(X=X, sid=torch.from_numpy(sorted_ids), off=torch.from_numpy(off), w=w).items()}
+    W13 = T.random_int4_weights(H, 2 * I, g, gen, experts=E)
+    d13 = [t.to(gpu) for t in W13]
+    act = torch.empty((P, I), dtype=torch.float16, device=gpu)
+    rt.call("tb_moe_w4a16_gate_up", rt.ptr(dev["X"]), rt.ptr(dev["sid"]), rt.ptr(dev["off"]), *map(rt.ptr, d13),
+            rt.ptr(act), Tk, k, E, H, I, g, rt.stream_handle(gpu))
+    torch.cuda.synchronize()
+    want = oracle.moe_gate_up(X.numpy(), sid, off, k, *(t.numpy() for t in W13), g)
+    got = act.cpu().numpy()[:len(sid)]
+    np.testing.assert_allclose(got.astype(np.float32), want[:len(sid)].astype(np.float32), atol=1e-2, rtol=1e-2)
+    if I % 64 or g > I:
+        return  # down needs K = I in whole groups
+    W2 = T.random_int4_weights(I, H, 64, gen, experts=E)
+    d2 = [t.to(gpu) for t in W2]
+    y = torch.full((P, H), float("nan"), dtype=torch.float16, device=gpu)
+    rt.call("tb_moe_w4a16_down", rt.ptr(act), rt.ptr(dev["sid"]), rt.ptr(dev["off"]), rt.ptr(dev["w"]),
+            *map(rt.ptr, d2), rt.ptr(y), P, E, I, H, 64, rt.stream_handle(gpu))
+    torch.cuda.synchronize()
+    want, written = oracle.moe_down(got, sid, off, w.numpy(), P, *(t.numpy() for t in W2), 64)
+    y = y.cpu().numpy()
+    np.testing.assert_allclose(y[written].astype(np.float32), want[written].astype(np.float32), atol=1e-2, rtol=1e-2)
+    assert np.isnan(y[~written].astype(np.float32)).all()

@@ -1,0 +1,28 @@
+"""The rule that picks a W4A16 tile (tilebench_amd/csrc/small_plan.h): the sizes
+of the GPU parity tests run the tile they are listed under."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from small_tile_cases import EXPERT_TILE_IDS, EXPERT_TILES
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _build(tmp_path):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path / "small_plan_pick")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "tilebench_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "small_plan_pick.cpp"), "-o", exe], check=True)
+    return exe
+
+
+def test_expert_tiles_picked(tmp_path):
+    exe = _build(tmp_path)
+    cases = [(tile, sum(rows), len(rows), N) for tile, cs in EXPERT_TILES.items() for rows, N, _, _ in cs]
+    args = [str(x) for _, *c in cases for x in c]
+    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
+    assert [int(g) for g in got] == [EXPERT_TILE_IDS[c[0]] for c in cases]

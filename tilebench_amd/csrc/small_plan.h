@@ -1,0 +1,54 @@
+// Which tile a W4A16 product runs on: host-only C++ (no HIP), shared with a CPU
+// check.
+//
+// A product's time is about its K steps times the time of one step of all its
+// tiles on 256 CUs.  Measured on MI355X (graph replays, K = 4096, us per K step
+// of 64): a 32 x 128 tile takes 0.25, 32 x 256 0.37, 64 x 256 0.42 - 0.56 (one
+// tile per CU - many), 256 x 256 0.9 - 1.9 (its MFMAs at the power cap).  Tiles
+// that share a CU share its VALU (the dequantisation bounds the small ones), so
+// their steps add up; a 256 x 256 tile fills a CU.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+namespace tb {
+namespace plan {
+
+enum ExpertTile { TILE_256 = 0, TILE_32x128, TILE_32x256, TILE_64x256 };
+
+// Tiles of `tm` rows for `rows` rows over `active` experts: half a tile of
+// padding per expert, at least one tile each.
+inline double expert_tile_rows(double rows, double active, double tm) {
+  return std::max(active, rows / tm + active / 2);
+}
+
+// The tile of a grouped, gate/up (N = 2 I columns of W13) or down product.  The
+// host knows the row count only, so at most `rows` experts have a tile and the
+// rows are taken as spread over them.  Measured (64 experts, top 8, H = 4096, I =
+// 704; gate/up + down us, this tile against 256 x 256): 1 token 23 + 8 (32 x
+// 128) against 84 + 18; 24 tokens 48 + 20 (32 x 256) against 164 + 56; 256
+// tokens 68 + 33 (64 x 256, 32 x 256) against 166 + 69; 1024 tokens 137 + 74
+// (64 x 256) against 191 + 104; 4096 tokens 445 + 265 (64 x 256) against 414 +
+// 251: the 256-row tiles stay there.
+inline ExpertTile pick_expert_tile(int64_t rows, int64_t experts, int64_t N) {
+  const double r = (double)rows, active = (double)std::min(rows, experts);
+  const double n128 = (double)((N + 127) / 128), n256 = (double)((N + 255) / 256);
+  const double big_n = (double)((N + 127) / 128) / 2;  // a last column tile of <= 128 columns is half a tile
+  auto load = [](double tiles) { return std::max(1.0, tiles / 256.0); };
+  const double c128 = 0.25 * load(expert_tile_rows(r, active, 32) * n128);
+  const double c256 = 0.37 * load(expert_tile_rows(r, active, 32) * n256);
+  const double tiles64 = expert_tile_rows(r, active, 64) * n256;
+  const double c64 = tiles64 <= 256 ? 0.42 + 0.14 * tiles64 / 256 : 0.56 * tiles64 / 256;
+  const double tiles_big = expert_tile_rows(r, active, 256) * big_n;
+  const double cbig = tiles_big <= 256 ? 0.9 : std::max(1.8, 1.88 * tiles_big / 256);
+  ExpertTile best = TILE_256;
+  double c = cbig;
+  if (c64 < c) best = TILE_64x256, c = c64;
+  if (c256 < c) best = TILE_32x256, c = c256;
+  if (c128 < c) best = TILE_32x128, c = c128;
+  return best;
+}
+
+}  // namespace plan
+}  // namespace tb

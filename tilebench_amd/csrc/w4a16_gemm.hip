@@ -53,6 +53,7 @@
 // the blocks resident on one XCD share A rows and W columns in its L2.
 #include "tb_common.h"
 #include "prefill_plan.h"
+#include "w4a16_small.h"
 #include "w4a16_tile.h"
 
 #include <algorithm>
@@ -1499,6 +1500,13 @@ extern "C" tb_status tb_moe_w4a16_grouped_gemm(const uint16_t* A, const uint8_t*
   TB_CHECK_ALIGN(scales, 16, "scales");
   TB_CHECK_ALIGN(zeros, 4, "zeros");
   TB_CHECK_ALIGN(Y, 16, "Y");
+  const auto tile = tb::plan::pick_expert_tile(R, experts, N);
+  if (tile != tb::plan::TILE_256)
+    return launch_experts_small("tb_moe_w4a16_grouped_gemm", T_PLAIN, tile,
+                                {reinterpret_cast<const _Float16*>(A), nullptr, offsets, nullptr, W,
+                                 reinterpret_cast<const _Float16*>(scales), zeros, reinterpret_cast<_Float16*>(Y), 0, 1,
+                                 R, (int)experts, (int)N, (int)K, (int)group},
+                                stream);
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(&w4a16_grouped), p8::LDS_BYTES, "tb_moe_w4a16_grouped_gemm")) return st;
   const int64_t tiles_n = (N + BN - 1) / BN;
   const int64_t tile_rows = (R + BM - 1) / BM + experts;  // upper bound on sum_e ceil(rows_e / 256)
@@ -1533,6 +1541,13 @@ extern "C" tb_status tb_moe_w4a16_gate_up(const uint16_t* X, const int32_t* sort
   TB_CHECK_ALIGN(S13, 16, "S13");
   TB_CHECK_ALIGN(Z13, 4, "Z13");
   TB_CHECK_ALIGN(act, 16, "act");
+  const auto tile = tb::plan::pick_expert_tile(pairs, experts, 2 * I);
+  if (tile != tb::plan::TILE_256)
+    return launch_experts_small(fn, T_GATE_UP, tile,
+                                {reinterpret_cast<const _Float16*>(X), sorted_ids, offsets, nullptr, W13,
+                                 reinterpret_cast<const _Float16*>(S13), Z13, reinterpret_cast<_Float16*>(act),
+                                 (int)tokens, (int)topk, pairs, (int)experts, (int)(2 * I), (int)H, (int)group},
+                                stream);
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(&moe_gate_up), p8::LDS_BYTES, fn)) return st;
   const int64_t tiles_n = (I + BN / 2 - 1) / (BN / 2);
   const int64_t tile_rows = (pairs + BM - 1) / BM + experts;
@@ -1565,6 +1580,13 @@ extern "C" tb_status tb_moe_w4a16_down(const uint16_t* act, const int32_t* sorte
   TB_CHECK_ALIGN(S2, 16, "S2");
   TB_CHECK_ALIGN(Z2, 4, "Z2");
   TB_CHECK_ALIGN(Y, 16, "Y");
+  const auto tile = tb::plan::pick_expert_tile(pairs, experts, H);
+  if (tile != tb::plan::TILE_256)
+    return launch_experts_small(fn, T_DOWN, tile,
+                                {reinterpret_cast<const _Float16*>(act), sorted_ids, offsets, topk_weights, W2,
+                                 reinterpret_cast<const _Float16*>(S2), Z2, reinterpret_cast<_Float16*>(Y), 0, 1, pairs,
+                                 (int)experts, (int)H, (int)I, (int)group},
+                                stream);
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(&moe_down), p8::LDS_BYTES, fn)) return st;
   const int64_t tiles_n = (H + BN - 1) / BN;
   const int64_t tile_rows = (pairs + BM - 1) / BM + experts;

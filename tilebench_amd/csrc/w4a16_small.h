@@ -1,0 +1,33 @@
+// Launchers of the small W4A16 tiles (w4a16_small.hip).
+#pragma once
+#include "small_plan.h"
+#include "w4a16_tile.h"
+
+namespace tb {
+namespace w4a16 {
+
+// One product per expert: rows of the row space (offsets[e] .. offsets[e + 1] is
+// expert e's) times W [K, N].  T_PLAIN: rows are A's and Y's.  T_GATE_UP: A is
+// X [tokens, K], row m reads token ids[m] / topk, W is W13 (N = 2 I) and Y
+// [rows, I].  T_DOWN: row m is scaled by weights[ids[m]] and stored at row
+// ids[m] of Y.
+struct ExpertArgs {
+  const _Float16* A;
+  const int* ids;
+  const int* offsets;
+  const float* weights;
+  const uint8_t* W;
+  const _Float16* S;
+  const uint8_t* Z;
+  _Float16* Y;
+  int tokens, topk;
+  int64_t rows;
+  int experts, N, K, group;
+};
+
+// Arguments checked by the caller (the limits of the 256-row kernels).
+tb_status launch_experts_small(const char* fn, TileMode mode, plan::ExpertTile tile, const ExpertArgs& a,
+                               hipStream_t stream);
+
+}  // namespace w4a16
+}  // namespace tb
