@@ -1,6 +1,7 @@
 // Prints the tile that tilebench_amd/csrc/small_plan.h picks for each
 // "rows experts N" triple on the command line (0: 256 rows, 1: 32 x 128,
-// 2: 32 x 256, 3: 64 x 256).
+// 2: 32 x 256, 3: 64 x 256); experts = 0 asks for the dense product of rows x N
+// (0: 256 x 256, 1: 64 x 64, 2: 64 x 128, 3: 64 x 256, 4: 128 x 256).
 // Build: g++ -O2 -std=c++17 -I tilebench_amd/csrc tests/native/small_plan_pick.cpp
 #include <cstdio>
 #include <cstdlib>
@@ -8,7 +9,9 @@
 #include "small_plan.h"
 
 int main(int argc, char** argv) {
-  for (int i = 1; i + 2 < argc; i += 3)
-    std::printf("%d\n", (int)tb::plan::pick_expert_tile(std::atoll(argv[i]), std::atoll(argv[i + 1]), std::atoll(argv[i + 2])));
+  for (int i = 1; i + 2 < argc; i += 3) {
+    const long long rows = std::atoll(argv[i]), experts = std::atoll(argv[i + 1]), N = std::atoll(argv[i + 2]);
+    std::printf("%d\n", experts ? (int)tb::plan::pick_expert_tile(rows, experts, N) : (int)tb::plan::pick_dense_tile(rows, N));
+  }
   return 0;
 }

@@ -1,12 +1,12 @@
 """GPU parity of the small W4A16 tiles (w4a16_small.hip): every tile of the
-grouped, gate/up and down products against the CPU oracle, and bit for bit
+dense, grouped, gate/up and down products against the CPU oracle, and bit for bit
 against the 256-row tiles on the same rows."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from small_tile_cases import EXPERT_TILES
+from small_tile_cases import DENSE_TILES, EXPERT_TILES
 from tilebench_amd import runtime as rt
 from tilebench_amd.data import tensors as T
 
@@ -97,3 +97,35 @@ def test_gate_up_and_down_tiles_match_oracle(gpu, Tk, E, k, H, I, g):
     y = y.cpu().numpy()
     np.testing.assert_allclose(y[written].astype(np.float32), want[written].astype(np.float32), atol=1e-2, rtol=1e-2)
     assert np.isnan(y[~written].astype(np.float32)).all()
+
+
+@pytest.mark.parametrize("tile", list(DENSE_TILES))
+def test_dense_tiles_match_oracle(gpu, tile):
+    from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
+
+    for M, K, N, G in DENSE_TILES[tile]:
+        _say("dense", tile, M, K, N, G)
+        A, p, s, z, G = T.generate_w4a16_gemm_inputs(M, K, N, G, seed=M + N, device="cpu")
+        Y = impl_hip.run(A.to(gpu), p.to(gpu), s.to(gpu), z.to(gpu), G)
+        torch.cuda.synchronize()
+        rows = np.unique(np.r_[np.arange(min(M, 96)), np.arange(max(0, M - 96), M)])
+        ref = oracle.w4a16_gemm(A.numpy()[rows], p.numpy(), s.numpy(), z.numpy(), G)
+        np.testing.assert_allclose(Y.cpu().numpy()[rows].astype(np.float32), ref.astype(np.float32), atol=1e-2,
+                                   rtol=1e-2)
+
+
+@pytest.mark.parametrize("M", [65, 500, 900])  # 64 x 128, 128 x 256 and 64 x 256 tiles
+def test_dense_rows_do_not_depend_on_the_tile(gpu, M):
+    """More than 64 rows: the first M rows alone give the bits they have in a
+    product of 256 x 256 tiles.  64 rows (K in four groups) are reproducible."""
+    from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
+
+    A, p, s, z, G = T.generate_w4a16_gemm_inputs(1024, 448, 11008 if M != 900 else 10752, 64, seed=3, device="cpu")
+    _say("dense rows", M)
+    A, p, s, z = (t.to(gpu) for t in (A, p, s, z))
+    big = impl_hip.run(A, p, s, z, G)
+    small = impl_hip.run(A[:M].contiguous(), p, s, z, G)
+    a, b = (impl_hip.run(A[:64].contiguous(), p, s, z, G) for _ in range(2))
+    torch.cuda.synchronize()
+    assert torch.equal(small.view(torch.int16), big[:M].view(torch.int16))
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))

@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from small_tile_cases import EXPERT_TILE_IDS, EXPERT_TILES
+from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -26,3 +26,11 @@ def test_expert_tiles_picked(tmp_path):
     args = [str(x) for _, *c in cases for x in c]
     got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
     assert [int(g) for g in got] == [EXPERT_TILE_IDS[c[0]] for c in cases]
+
+
+def test_dense_tiles_picked(tmp_path):
+    exe = _build(tmp_path)
+    cases = [(tile, M, 0, N) for tile, cs in DENSE_TILES.items() for M, _, N, _ in cs]
+    args = [str(x) for _, *c in cases for x in c]
+    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
+    assert [int(g) for g in got] == [DENSE_TILE_IDS[c[0]] for c in cases]

@@ -50,5 +50,34 @@ inline ExpertTile pick_expert_tile(int64_t rows, int64_t experts, int64_t N) {
   return best;
 }
 
+enum DenseTile { DENSE_256 = 0, DENSE_64x64_K4, DENSE_64x128, DENSE_64x256, DENSE_128x256 };
+
+// The tile of a dense product of more than 16 rows, by the same estimate (us per
+// K step, measured at K = 4096 and 11008 on 43 - 1376 tiles).  Up to 64 rows
+// 64-column tiles of four K groups put a product on every CU that has columns
+// for it: 48 rows x 11008 columns 15 us against 25 (64 x 128), 30 (64 x 256)
+// and 62 (256 x 256).  128 x 11008 (K = 4096): 64 x 128 25 us, 64 x 256 31, 128
+// x 256 42, 256 x 256 63; 512 x 11008: 61 / 59 / 52 / 71; 1024 x 11008: 116 /
+// 101 / 106 / 95; 500 x 4096 (K = 11008): 65 / 78 / 106 / 160.
+inline DenseTile pick_dense_tile(int64_t M, int64_t N) {
+  auto tiles = [&](int64_t tm, int64_t tn) { return (double)((M + tm - 1) / tm * ((N + tn - 1) / tn)) / 256.0; };
+  // x: tiles per CU
+  auto c64 = [](double x) { return 0.18 * std::max(1.0, x); };
+  auto c128 = [](double x) { return x <= 1 ? 0.30 + 0.05 * x : std::max(0.5, 0.32 * x); };
+  auto c256 = [](double x) { return x <= 1 ? 0.40 + 0.10 * x : std::max(0.83, 0.55 * x); };
+  auto c128x256 = [](double x) { return x <= 1 ? 0.56 + 0.25 * x : std::max(1.56, x); };  // one tile per CU
+  auto cbig = [](double x) { return x <= 1 ? 0.80 + 0.85 * x : std::max(2.66, 1.74 * x); };
+  DenseTile best = DENSE_256;
+  double c = cbig(tiles(256, 256));
+  auto take = [&](DenseTile t, double cost) {
+    if (cost < c) best = t, c = cost;
+  };
+  take(DENSE_128x256, c128x256(tiles(128, 256)));
+  take(DENSE_64x256, c256(tiles(64, 256)));
+  take(DENSE_64x128, c128(tiles(64, 128)));
+  if (M <= 64) take(DENSE_64x64_K4, c64(tiles(64, 64)));
+  return best;
+}
+
 }  // namespace plan
 }  // namespace tb

@@ -1349,7 +1349,8 @@ static tb_status check_dense_args(const char* fn, const uint16_t* A, const uint8
 
 // Launch of the dense W4A16 GEMM after the checks: the split-K decode kernel
 // for M <= 16 (counters at `workspace`, fp32 partials DEC_COUNTER_BYTES past
-// it), the MFMA prefill kernel otherwise.
+// it), otherwise the MFMA prefill kernel or, where its 256 x 256 tiles leave
+// CUs idle, a small tile (small_plan.h).
 // How the dense prefill covers the output (256-row tiles over the first
 // n_split tile columns, 192-row tiles over the rest): tb::plan::plan_prefill,
 // prefill_plan.h, a closed-form evaluation of the greedy schedule per split.
@@ -1375,6 +1376,12 @@ static tb_status launch_dense(const char* fn, const uint16_t* A, const uint8_t* 
                          reinterpret_cast<_Float16*>(Y), partials, counters, (int)M, (int)N, (int)K, (int)group, splits);
     return tb::launch_status(fn);
   }
+  const auto tile = tb::plan::pick_dense_tile(M, N);
+  if (tile != tb::plan::DENSE_256)
+    return launch_dense_small(fn, tile,
+                              {reinterpret_cast<const _Float16*>(A), W, reinterpret_cast<const _Float16*>(scales),
+                               zeros, reinterpret_cast<_Float16*>(Y), (int)M, (int)N, (int)K, (int)group},
+                              stream);
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(&w4a16_prefill), p8::LDS_BYTES, fn)) return st;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
   const PrefillPlan pl = plan_prefill((int)M, tiles_m, tiles_n, device_cus());

@@ -27,7 +27,10 @@
 // dequantisation to fp16, the same v_mfma_f32_32x32x16_f16 operands in the same
 // K order per output element, the same epilogue roundings; results are
 // bit-identical to them, so neither the choice of tile nor the call that uses
-// it shows in an output.  Nothing splits K, so no workspace is needed.
+// it shows in an output.  Only the dense product of at most 64 rows (S64x64k4)
+// splits K, over four groups of wavefronts of one block whose fp32 sums are
+// added through LDS in group order: reproducible, but not the unsplit order.
+// No workspace is needed.
 #include "w4a16_small.h"
 
 #include <type_traits>
@@ -71,6 +74,9 @@ struct Shape {
 typedef Shape<1, 2, true, 1, 3> S32x128;
 typedef Shape<1, 4, false, 1, 3> S32x256;
 typedef Shape<2, 4, false, 1, 3> S64x256;
+typedef Shape<2, 1, true, 1, 3, 4> S64x64k4;
+typedef Shape<2, 2, true, 1, 4> S64x128;
+typedef Shape<4, 4, false, 1, 3> S128x256;
 
 // 16-byte chunk c of packed row r sits at slot c ^ wswz(r): the eight rows of a
 // transposing read (and its two chunks) then sit in different banks.
@@ -478,6 +484,24 @@ __device__ __forceinline__ void tile(uint8_t* __restrict__ lds, const _Float16* 
   }
 }
 
+// Blocks go round-robin over the 8 XCDs: XCD x takes a contiguous run of tiles,
+// so that the blocks of one L2 share W lines and A rows.
+__device__ __forceinline__ int xcd_run(int bid, int nb) {
+  const int x = bid & 7, q = nb >> 3, rem = nb & 7;
+  return x * q + min(x, rem) + (bid >> 3);
+}
+
+// Dense: tiles in column order, all row tiles of a column together.
+template <class C, bool WIDE>
+__global__ void __launch_bounds__(C::THREADS, C::MIN_WAVES)
+    w4a16_dense(const _Float16* __restrict__ A, const uint8_t* __restrict__ W, const _Float16* __restrict__ S,
+                const uint8_t* __restrict__ Z, _Float16* __restrict__ Y, int M, int N, int K, int group, int tiles_m) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int idx = xcd_run(blockIdx.x, gridDim.x);
+  const int nt = idx / tiles_m, mt = idx - nt * tiles_m;
+  tile<C, WIDE, T_PLAIN>(lds, A, W, S, Z, Y, M, N, K, group, mt * C::TM, nt * C::TN, M, RowMap{});
+}
+
 // Grouped, gate/up and down products: the kernels of w4a16_gemm.hip on small
 // tiles (rows: pairs; A is X for the gate/up projection).
 template <class C, bool WIDE, int MODE>
@@ -501,6 +525,17 @@ __global__ void __launch_bounds__(C::THREADS, C::MIN_WAVES)
                       Z + e * zstride, MODE == T_DOWN ? Y : Y + (int64_t)m0 * ldy, m_end - m0, N, K, group, 0,
                       nt * C::TN, MODE == T_GATE_UP ? tokens : m_end - m0, rm);
 }
+template <class C, bool WIDE>
+tb_status launch_dense_shape(const char* fn, const DenseArgs& a, hipStream_t stream) {
+  auto kern = &w4a16_dense<C, WIDE>;
+  if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(kern), C::LDS_BYTES, fn)) return st;
+  const int64_t tiles_m = (a.M + C::TM - 1) / C::TM, tiles_n = (a.N + C::TN - 1) / C::TN;
+  TB_CHECK_ARG(tiles_m * tiles_n < (1ll << 31), "%s: problem too large", fn);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(C::THREADS), C::LDS_BYTES, stream, a.A, a.W, a.S,
+                     a.Z, a.Y, a.M, a.N, a.K, a.group, (int)tiles_m);
+  return tb::launch_status(fn);
+}
+
 template <class C, bool WIDE, int MODE>
 tb_status launch_shape(const char* fn, const ExpertArgs& a, hipStream_t stream) {
   auto kern = &w4a16_experts<C, WIDE, MODE>;
@@ -530,6 +565,21 @@ tb_status launch_mode(const char* fn, plan::ExpertTile tile, const ExpertArgs& a
   }
 }
 }  // namespace sm
+
+tb_status launch_dense_small(const char* fn, plan::DenseTile tile, const DenseArgs& a, hipStream_t stream) {
+  using namespace sm;
+  const bool wide = tb::aligned(a.W, 16) && a.N % 32 == 0;
+  switch (tile) {
+    case plan::DENSE_64x64_K4:
+      return wide ? launch_dense_shape<S64x64k4, true>(fn, a, stream) : launch_dense_shape<S64x64k4, false>(fn, a, stream);
+    case plan::DENSE_64x128:
+      return wide ? launch_dense_shape<S64x128, true>(fn, a, stream) : launch_dense_shape<S64x128, false>(fn, a, stream);
+    case plan::DENSE_64x256:
+      return wide ? launch_dense_shape<S64x256, true>(fn, a, stream) : launch_dense_shape<S64x256, false>(fn, a, stream);
+    default:
+      return wide ? launch_dense_shape<S128x256, true>(fn, a, stream) : launch_dense_shape<S128x256, false>(fn, a, stream);
+  }
+}
 
 tb_status launch_experts_small(const char* fn, TileMode mode, plan::ExpertTile tile, const ExpertArgs& a,
                                hipStream_t stream) {
