@@ -1,7 +1,8 @@
 // Prints the tile that tilebench_amd/csrc/small_plan.h picks for each
 // "rows experts N" triple on the command line (0: 256 rows, 1: 32 x 128,
 // 2: 32 x 256, 3: 64 x 256); experts = 0 asks for the dense product of rows x N
-// (0: 256 x 256, 1: 64 x 64, 2: 64 x 128, 3: 64 x 256, 4: 128 x 256).
+// (0: 256 x 256, 1: 64 x 64, 2: 64 x 128, 3: 64 x 256, 4: 128 x 256), experts =
+// -K / -K - 1 for the rows per block of the row- / block-scaled fp8 product.
 // Build: g++ -O2 -std=c++17 -I tilebench_amd/csrc tests/native/small_plan_pick.cpp
 #include <cstdio>
 #include <cstdlib>
@@ -11,7 +12,12 @@
 int main(int argc, char** argv) {
   for (int i = 1; i + 2 < argc; i += 3) {
     const long long rows = std::atoll(argv[i]), experts = std::atoll(argv[i + 1]), N = std::atoll(argv[i + 2]);
-    std::printf("%d\n", experts ? (int)tb::plan::pick_expert_tile(rows, experts, N) : (int)tb::plan::pick_dense_tile(rows, N));
+    int pick;
+    if (experts < 0)
+      pick = tb::plan::pick_fp8_rows(rows, N, -experts / 128 * 128, experts % 128 != 0);
+    else
+      pick = experts ? (int)tb::plan::pick_expert_tile(rows, experts, N) : (int)tb::plan::pick_dense_tile(rows, N);
+    std::printf("%d\n", pick);
   }
   return 0;
 }

@@ -1,4 +1,4 @@
-"""Sizes that run each W4A16 tile (tilebench_amd/csrc/small_plan.h), shared by
+"""Sizes that run each W4A16 and scaled fp8 tile (tilebench_amd/csrc/small_plan.h), shared by
 the CPU check of the rule and the GPU parity tests."""
 
 #: tile -> (rows per expert, N of the product, K, group): rows on both sides of
@@ -22,3 +22,12 @@ DENSE_TILES = {
     "256": [(1024, 192, 11008, 64)],
 }
 DENSE_TILE_IDS = {"256": 0, "64x64": 1, "64x128": 2, "64x256": 3, "128x256": 4}
+
+#: rows per block -> (M, N, K) of the scaled fp8 products (both scalings): ragged
+#: rows and columns, one K step, fewer K steps than wavefronts, odd step counts
+FP8_ROWS = {
+    32: [(1, 8, 128), (33, 200, 384), (31, 2112, 1408), (70, 136, 896)],
+    64: [(64, 8192, 384), (126, 4000, 640)],
+    128: [(256, 4096, 640), (250, 4072, 896)],
+    0: [(513, 8192, 256), (1024, 4104, 1152)],
+}

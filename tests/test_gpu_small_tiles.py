@@ -1,12 +1,13 @@
 """GPU parity of the small W4A16 tiles (w4a16_small.hip): every tile of the
 dense, grouped, gate/up and down products against the CPU oracle, and bit for bit
-against the 256-row tiles on the same rows."""
+against the 256-row tiles on the same rows; and of the few-row scaled fp8
+products (fp8_small.hip) against the oracle."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from small_tile_cases import DENSE_TILES, EXPERT_TILES
+from small_tile_cases import DENSE_TILES, EXPERT_TILES, FP8_ROWS
 from tilebench_amd import runtime as rt
 from tilebench_amd.data import tensors as T
 
@@ -129,3 +130,26 @@ def test_dense_rows_do_not_depend_on_the_tile(gpu, M):
     torch.cuda.synchronize()
     assert torch.equal(small.view(torch.int16), big[:M].view(torch.int16))
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("rows", list(FP8_ROWS))
+@pytest.mark.parametrize("scaling", ["row", "block"])
+def test_fp8_rows_match_oracle(gpu, rows, scaling):
+    """bf16 within the operators' 1e-2, and reproducible bit for bit."""
+    if scaling == "row":
+        from tilebench_amd.benchmarks.operators.fp8_scaled_gemm import impl_hip
+        gen, ref_gemm = T.generate_fp8_scaled_gemm_inputs, oracle.fp8_scaled_gemm
+    else:
+        from tilebench_amd.benchmarks.operators.fp8_block_scaled_gemm import impl_hip
+        gen, ref_gemm = T.generate_fp8_block_scaled_gemm_inputs, oracle.fp8_block_gemm
+    for M, N, K in FP8_ROWS[rows]:
+        _say("fp8", scaling, rows, M, N, K)
+        Aq, W, sa, sw = gen(M, N, K, seed=M + N, device="cpu")
+        d = [t.to(gpu) for t in (Aq, W, sa, sw)]
+        Y, again = impl_hip.run(*d), impl_hip.run(*d)
+        torch.cuda.synchronize()
+        r = np.unique(np.r_[np.arange(min(M, 70)), np.arange(max(0, M - 70), M)])
+        s = sa.numpy()[r] if scaling == "row" else sa.numpy()[:, r]
+        ref = ref_gemm(Aq.view(torch.uint8).numpy()[r], W.contiguous().view(torch.uint8).numpy(), s, sw.numpy())
+        np.testing.assert_allclose(Y.float().cpu().numpy()[r], oracle.bf16_bits_to_f32(ref), atol=1e-2, rtol=1e-2)
+        assert torch.equal(Y.view(torch.int16), again.view(torch.int16))

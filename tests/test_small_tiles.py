@@ -1,4 +1,4 @@
-"""The rule that picks a W4A16 tile (tilebench_amd/csrc/small_plan.h): the sizes
+"""The rules that pick a W4A16 or fp8 tile (tilebench_amd/csrc/small_plan.h): the sizes
 of the GPU parity tests run the tile they are listed under."""
 import os
 import shutil
@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES
+from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES, FP8_ROWS
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -34,3 +34,11 @@ def test_dense_tiles_picked(tmp_path):
     args = [str(x) for _, *c in cases for x in c]
     got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
     assert [int(g) for g in got] == [DENSE_TILE_IDS[c[0]] for c in cases]
+
+
+def test_fp8_rows_picked(tmp_path):
+    exe = _build(tmp_path)
+    cases = [(rows, M, -K - blk, N) for rows, cs in FP8_ROWS.items() for M, N, K in cs for blk in (0, 1)]
+    args = [str(x) for _, *c in cases for x in c]
+    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
+    assert [int(g) for g in got] == [c[0] for c in cases]

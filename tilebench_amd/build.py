@@ -40,11 +40,12 @@ HIPCC_FLAGS = [
 ]
 
 
-#: extra flags for single sources.  fp8_block.hip: its MFMA results feed VALU
-#: FMAs every K step, so they are kept in VGPRs (the default puts MFMA results
+#: extra flags for single sources.  fp8_block.hip, fp8_small.hip: their MFMA
+#: results feed VALU FMAs every K step, so they are kept in VGPRs (the default puts MFMA results
 #: in AGPRs, which costs a v_accvgpr_read per element before each FMA).
 FILE_FLAGS = {
     "fp8_block.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "fp8_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

@@ -31,6 +31,7 @@
 // operands, permuted so that a lane reads its four rows' scales with one
 // 16-byte LDS read; the tile's two columns of weight scales (K/128 values
 // each) are loaded once at the start.
+#include "fp8_small.h"
 #include "tb_common.h"
 #include "fp8_codec.h"
 
@@ -457,5 +458,7 @@ extern "C" tb_status tb_fp8_block_gemm(const uint8_t* Aq, const uint8_t* WqT, co
   TB_CHECK_ALIGN(sa, 4, "sa");
   TB_CHECK_ALIGN(sw, 4, "sw");
   TB_CHECK_ALIGN(Y, 16, "Y");
+  if (const int rows = tb::plan::pick_fp8_rows(M, N, K, true))
+    return tb::fp8s::launch_skinny("tb_fp8_block_gemm", rows, true, {Aq, WqT, sa, sw, Y, (int)M, (int)N, (int)K}, stream);
   return launch_block<kLaunchBN, kLaunchWaves, kLaunchStages>(Aq, WqT, sa, sw, Y, M, N, K, stream);
 }

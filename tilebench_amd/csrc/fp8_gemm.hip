@@ -28,6 +28,7 @@
 // accumulator elements; the epilogue scales, rounds to bf16, stages the tile
 // in LDS with 8-byte writes and stores 16-byte row chunks.  Tiles are numbered
 // XCD-aware as in the W4A16 kernel.
+#include "fp8_small.h"
 #include "tb_common.h"
 
 #include <type_traits>
@@ -320,6 +321,8 @@ extern "C" tb_status tb_fp8_scaled_gemm(const uint8_t* Aq, const uint8_t* WqT, c
   TB_CHECK_ALIGN(Aq, 16, "Aq");
   TB_CHECK_ALIGN(WqT, 16, "WqT");
   TB_CHECK_ALIGN(Y, 16, "Y");
+  if (const int rows = tb::plan::pick_fp8_rows(M, N, K, false))
+    return tb::fp8s::launch_skinny("tb_fp8_scaled_gemm", rows, false, {Aq, WqT, sa, sw, Y, (int)M, (int)N, (int)K}, stream);
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(&fp8_gemm_kernel), LDS_BYTES, "tb_fp8_scaled_gemm"))
     return st;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);

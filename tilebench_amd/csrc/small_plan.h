@@ -1,7 +1,7 @@
-// Which tile a W4A16 product runs on: host-only C++ (no HIP), shared with a CPU
-// check.
+// Which tile a W4A16 or scaled fp8 product runs on: host-only C++ (no HIP),
+// shared with a CPU check.
 //
-// A product's time is about its K steps times the time of one step of all its
+// A W4A16 product's time is about its K steps times the time of one step of all its
 // tiles on 256 CUs.  Measured on MI355X (graph replays, K = 4096, us per K step
 // of 64): a 32 x 128 tile takes 0.25, 32 x 256 0.37, 64 x 256 0.42 - 0.56 (one
 // tile per CU - many), 256 x 256 0.9 - 1.9 (its MFMAs at the power cap).  Tiles
@@ -76,6 +76,30 @@ inline DenseTile pick_dense_tile(int64_t M, int64_t N) {
   take(DENSE_64x256, c256(tiles(64, 256)));
   take(DENSE_64x128, c128(tiles(64, 128)));
   if (M <= 64) take(DENSE_64x64_K4, c64(tiles(64, 64)));
+  return best;
+}
+
+// Rows per block of the few-row scaled fp8 GEMM (32, 64 or 128; 32 columns per
+// block), or 0 for the 256 x 256 tiles.  A few-row block is bound by its CU's
+// loads: measured about 1.5 us + (its rows of A and W) x K / 33 KB per us, blocks
+// that share a CU in turn (8192 x 8192 weights: 1 row 12.4 us, 32 rows 17.4, 64
+// rows 24.6 in 64-row blocks and 31.6 in 32-row ones; 128 x 4096 x 4096: 17.8 /
+// 14.1 / 21.9 us in 32- / 64- / 128-row blocks).  A round of 256 x 256 tiles takes
+// 5 us + 0.9 us per 128 bytes of K on a few CUs, 1.55 us on all (block scales:
+// 1.45 and 1.9): 32 rows 65 us, 256 x 4096 x 4096 38 us (few-row 22.5), 512 x 4096
+// x 4096 39 us (few-row 40).
+inline int pick_fp8_rows(int64_t M, int64_t N, int64_t K, bool block_scaled) {
+  const double steps = (double)K / 128;
+  const double x = (double)((M + 255) / 256 * ((N + 255) / 256)) / 256;
+  const double few = block_scaled ? 1.45 : 0.9, all = block_scaled ? 1.9 : 1.55;
+  double c = x <= 1 ? 5 + steps * (few + (all - few) * x) : (5 + steps * all) * x;
+  int best = 0;
+  for (int rows : {32, 64, 128}) {
+    const double blocks = (double)((M + rows - 1) / rows * ((N + 31) / 32));
+    const double rounds = (double)(int64_t)((blocks + 255) / 256);
+    const double t = rounds * (1.5 + (double)(std::min<int64_t>(rows, M) + 32) * (double)K / 33e3);
+    if (t < c) best = rows, c = t;
+  }
   return best;
 }
 
