@@ -69,7 +69,8 @@ def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torc
         _last_config = {"kernel": "w4a16_slab_decode", "layout": "slabs", "cols_per_block": 64, "waves": 16}
         return Y
     need = ctypes.c_int64(0)
-    rt.call("tb_w4a16_workspace_size", M, N, K, group, ctypes.byref(need))
+    if M <= 16:  # only the split-K decode has a workspace
+        rt.call("tb_w4a16_workspace_size", M, N, K, group, ctypes.byref(need))
     ws = rt.workspace(need.value, A.device, stream)
     rt.call("tb_w4a16_gemm", A.data_ptr(), packed.data_ptr(), scales.data_ptr(), zeros.data_ptr(), Y.data_ptr(),
             M, N, K, group, rt.ptr(ws), need.value, stream)
