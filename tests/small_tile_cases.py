@@ -23,11 +23,14 @@ DENSE_TILES = {
 }
 DENSE_TILE_IDS = {"256": 0, "64x64": 1, "64x128": 2, "64x256": 3, "128x256": 4}
 
-#: rows per block -> (M, N, K) of the scaled fp8 products (both scalings): ragged
-#: rows and columns, one K step, fewer K steps than wavefronts, odd step counts
-FP8_ROWS = {
-    32: [(1, 8, 128), (33, 200, 384), (31, 2112, 1408), (70, 136, 896)],
-    64: [(64, 8192, 384), (126, 4000, 640)],
-    128: [(256, 4096, 640), (250, 4072, 896)],
-    0: [(513, 8192, 256), (1024, 4104, 1152)],
+#: tile -> (M, N, K) of the scaled fp8 products (both scalings): ragged rows and
+#: columns, one K step, fewer K steps than wavefronts or ring stages, odd step
+#: counts, one and several tiles per CU
+FP8_TILES = {
+    "32x32": [(1, 8, 128), (31, 2112, 1408), (16, 8184, 896)],
+    "64x64": [(65, 4000, 640), (126, 4104, 128), (200, 2112, 1152)],
+    "64x128": [(126, 8200, 128), (300, 5000, 384)],
+    "128x128": [(512, 4104, 640), (600, 8200, 1024)],
+    "256": [(1024, 8200, 1152)],
 }
+FP8_TILE_IDS = {"256": 0, "32x32": 1, "64x64": 2, "64x128": 3, "128x128": 4}

@@ -1,13 +1,13 @@
 """GPU parity of the small W4A16 tiles (w4a16_small.hip): every tile of the
 dense, grouped, gate/up and down products against the CPU oracle, and bit for bit
-against the 256-row tiles on the same rows; and of the few-row scaled fp8
-products (fp8_small.hip) against the oracle."""
+against the 256-row tiles on the same rows; and of the small-tile scaled
+fp8 products (fp8_small.hip) against the oracle."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from small_tile_cases import DENSE_TILES, EXPERT_TILES, FP8_ROWS
+from small_tile_cases import DENSE_TILES, EXPERT_TILES, FP8_TILES
 from tilebench_amd import runtime as rt
 from tilebench_amd.data import tensors as T
 
@@ -132,9 +132,9 @@ def test_dense_rows_do_not_depend_on_the_tile(gpu, M):
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
-@pytest.mark.parametrize("rows", list(FP8_ROWS))
+@pytest.mark.parametrize("tile", list(FP8_TILES))
 @pytest.mark.parametrize("scaling", ["row", "block"])
-def test_fp8_rows_match_oracle(gpu, rows, scaling):
+def test_fp8_tiles_match_oracle(gpu, tile, scaling):
     """bf16 within the operators' 1e-2, and reproducible bit for bit."""
     if scaling == "row":
         from tilebench_amd.benchmarks.operators.fp8_scaled_gemm import impl_hip
@@ -142,8 +142,8 @@ def test_fp8_rows_match_oracle(gpu, rows, scaling):
     else:
         from tilebench_amd.benchmarks.operators.fp8_block_scaled_gemm import impl_hip
         gen, ref_gemm = T.generate_fp8_block_scaled_gemm_inputs, oracle.fp8_block_gemm
-    for M, N, K in FP8_ROWS[rows]:
-        _say("fp8", scaling, rows, M, N, K)
+    for M, N, K in FP8_TILES[tile]:
+        _say("fp8", scaling, tile, M, N, K)
         Aq, W, sa, sw = gen(M, N, K, seed=M + N, device="cpu")
         d = [t.to(gpu) for t in (Aq, W, sa, sw)]
         Y, again = impl_hip.run(*d), impl_hip.run(*d)

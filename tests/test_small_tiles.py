@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES, FP8_ROWS
+from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES, FP8_TILE_IDS, FP8_TILES
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -36,9 +36,9 @@ def test_dense_tiles_picked(tmp_path):
     assert [int(g) for g in got] == [DENSE_TILE_IDS[c[0]] for c in cases]
 
 
-def test_fp8_rows_picked(tmp_path):
+def test_fp8_tiles_picked(tmp_path):
     exe = _build(tmp_path)
-    cases = [(rows, M, -K - blk, N) for rows, cs in FP8_ROWS.items() for M, N, K in cs for blk in (0, 1)]
+    cases = [(tile, M, -K - blk, N) for tile, cs in FP8_TILES.items() for M, N, K in cs for blk in (0, 1)]
     args = [str(x) for _, *c in cases for x in c]
     got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-    assert [int(g) for g in got] == [c[0] for c in cases]
+    assert [int(g) for g in got] == [FP8_TILE_IDS[c[0]] for c in cases]

@@ -458,7 +458,8 @@ extern "C" tb_status tb_fp8_block_gemm(const uint8_t* Aq, const uint8_t* WqT, co
   TB_CHECK_ALIGN(sa, 4, "sa");
   TB_CHECK_ALIGN(sw, 4, "sw");
   TB_CHECK_ALIGN(Y, 16, "Y");
-  if (const int rows = tb::plan::pick_fp8_rows(M, N, K, true))
-    return tb::fp8s::launch_skinny("tb_fp8_block_gemm", rows, true, {Aq, WqT, sa, sw, Y, (int)M, (int)N, (int)K}, stream);
+  const auto tile = tb::plan::pick_fp8_tile(M, N, K, true);
+  if (tile != tb::plan::FP8_256)
+    return tb::fp8s::launch_small("tb_fp8_block_gemm", tile, true, {Aq, WqT, sa, sw, Y, (int)M, (int)N, (int)K}, stream);
   return launch_block<kLaunchBN, kLaunchWaves, kLaunchStages>(Aq, WqT, sa, sw, Y, M, N, K, stream);
 }

@@ -321,8 +321,9 @@ extern "C" tb_status tb_fp8_scaled_gemm(const uint8_t* Aq, const uint8_t* WqT, c
   TB_CHECK_ALIGN(Aq, 16, "Aq");
   TB_CHECK_ALIGN(WqT, 16, "WqT");
   TB_CHECK_ALIGN(Y, 16, "Y");
-  if (const int rows = tb::plan::pick_fp8_rows(M, N, K, false))
-    return tb::fp8s::launch_skinny("tb_fp8_scaled_gemm", rows, false, {Aq, WqT, sa, sw, Y, (int)M, (int)N, (int)K}, stream);
+  const auto tile = tb::plan::pick_fp8_tile(M, N, K, false);
+  if (tile != tb::plan::FP8_256)
+    return tb::fp8s::launch_small("tb_fp8_scaled_gemm", tile, false, {Aq, WqT, sa, sw, Y, (int)M, (int)N, (int)K}, stream);
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(&fp8_gemm_kernel), LDS_BYTES, "tb_fp8_scaled_gemm"))
     return st;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);

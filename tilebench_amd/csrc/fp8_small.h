@@ -1,4 +1,4 @@
-// Launcher of the few-row scaled fp8 GEMM (fp8_small.hip).
+// Launcher of the small-tile scaled fp8 GEMMs (fp8_small.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -20,8 +20,7 @@ struct Fp8Args {
   int M, N, K;
 };
 
-// rows: 32, 64 or 128 (plan::pick_fp8_rows).
-tb_status launch_skinny(const char* fn, int rows, bool block_scaled, const Fp8Args& a, hipStream_t stream);
+tb_status launch_small(const char* fn, plan::Fp8Tile tile, bool block_scaled, const Fp8Args& a, hipStream_t stream);
 
 }  // namespace fp8s
 }  // namespace tb

@@ -95,12 +95,12 @@ __device__ __forceinline__ void tile(uint8_t* __restrict__ lds, const _Float16* 
   // W DMA instructions per step: 1 KiB (WIDE) or 256 bytes each
   constexpr int WTOT = C::W_ST / (WIDE ? 1024 : 256);
   constexpr int WI = WTOT / WAVES > 0 ? WTOT / WAVES : 1;
-  // WIDE with CW = 1 has two W instructions: of four wavefronts the first two
-  // issue them and the others fetch the scales and zero-points; otherwise the
-  // first ones do both (the rest's scale DMA lands in the pad, so that every
-  // wavefront counts the same)
+  // with fewer W instructions than wavefronts the first ones issue them and the
+  // next ones fetch the scales and zero-points; otherwise the first ones do both
+  // (the rest's scale DMA lands in the pad, so that every wavefront counts the
+  // same)
   constexpr bool SHARED = WTOT < WAVES;
-  static_assert(SHARED ? WTOT == 2 && WAVES == 4 : WTOT % WAVES == 0, "W DMA split");
+  static_assert(SHARED || WTOT % WAVES == 0, "W DMA split");
   constexpr int PER = AI + WI + (SHARED ? 0 : 1);  // DMAs per wavefront and step
   static_assert(PER * (ST - 1) < 64, "vmcnt range");
   const int t = threadIdx.x, lane = t & 63, h = lane >> 5, j = lane & 31;
@@ -165,7 +165,7 @@ __device__ __forceinline__ void tile(uint8_t* __restrict__ lds, const _Float16* 
   }
   // scales (4-byte DMAs of 128 columns, lane L columns 2L, 2L + 1) and
   // zero-points (lane L bytes 4L .. 4L + 3) of a step's group
-  constexpr int S_WAVE = SHARED ? 2 : 0, Z_WAVE = S_WAVE + C::SW;
+  constexpr int S_WAVE = SHARED ? WTOT : 0, Z_WAVE = S_WAVE + C::SW;
   static_assert(Z_WAVE < WAVES, "a wavefront for the zero-points");
   const bool zw = w == Z_WAVE;
   uint32_t sz_off = OOB, sz_lds = C::PAD_OFF;
