@@ -1,4 +1,4 @@
-"""Sizes that run each W4A16 and scaled fp8 tile (tilebench_amd/csrc/small_plan.h), shared by
+"""Sizes that run each W4A16, scaled fp8 and plain-product tile (tilebench_amd/csrc/small_plan.h), shared by
 the CPU check of the rule and the GPU parity tests."""
 
 #: tile -> (rows per expert, N of the product, K, group): rows on both sides of
@@ -34,3 +34,13 @@ FP8_TILES = {
     "256": [(1024, 8200, 1152)],
 }
 FP8_TILE_IDS = {"256": 0, "32x32": 1, "64x64": 2, "64x128": 3, "128x128": 4}
+
+#: tile -> (M, N, bytes of K per row) of the plain products: ragged rows and
+#: columns, one K step, odd step counts, one and several tiles per CU
+NT_TILES = {
+    "64x64": [(1, 8, 128), (65, 1000, 640), (100, 4104, 1152)],
+    "64x128": [(513, 2056, 640), (300, 5000, 384)],
+    "128x128": [(1000, 2104, 1152), (1100, 5000, 640)],
+    "256": [(4096, 4104, 1152)],
+}
+NT_TILE_IDS = {"256": 0, "64x64": 1, "64x128": 2, "128x128": 3}

@@ -1,13 +1,13 @@
 """GPU parity of the small W4A16 tiles (w4a16_small.hip): every tile of the
 dense, grouped, gate/up and down products against the CPU oracle, and bit for bit
 against the 256-row tiles on the same rows; and of the small-tile scaled
-fp8 products (fp8_small.hip) against the oracle."""
+fp8 (fp8_small.hip) and plain products (nt_gemm.hip) against the oracle."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from small_tile_cases import DENSE_TILES, EXPERT_TILES, FP8_TILES
+from small_tile_cases import DENSE_TILES, EXPERT_TILES, FP8_TILES, NT_TILES
 from tilebench_amd import runtime as rt
 from tilebench_amd.data import tensors as T
 
@@ -153,3 +153,54 @@ def test_fp8_tiles_match_oracle(gpu, tile, scaling):
         ref = ref_gemm(Aq.view(torch.uint8).numpy()[r], W.contiguous().view(torch.uint8).numpy(), s, sw.numpy())
         np.testing.assert_allclose(Y.float().cpu().numpy()[r], oracle.bf16_bits_to_f32(ref), atol=1e-2, rtol=1e-2)
         assert torch.equal(Y.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.parametrize("tile", list(NT_TILES))
+@pytest.mark.parametrize("dt", ["fp16", "fp32", "fp8", "int8"])
+def test_plain_product_tiles_match_oracle(gpu, tile, dt):
+    """Every type on every tile, at the tolerances of the products' own tests
+    (fp32 within 1e-4 of the float64 product, int8 exact, e4m3 codes equal on
+    99.5 % and never more than a step apart)."""
+    from tilebench_amd.benchmarks.operators.matmul_fp32_fp16_fp8 import impl_hip as mm
+    from tilebench_amd.benchmarks.operators.matmul_int8 import impl_hip as mi
+
+    for M, N, Kb in NT_TILES[tile]:
+        # elements of K whose GEMM row has Kb bytes (fp32: three bf16 terms, K % 64 == 0)
+        K = {"fp16": Kb // 2, "fp32": max(64, Kb // 6 // 64 * 64), "fp8": Kb, "int8": Kb}[dt]
+        _say("plain", dt, tile, M, N, K)
+        r = np.unique(np.r_[np.arange(min(M, 40)), np.arange(max(0, M - 40), M)])
+        if dt == "int8":
+            a, b = T.generate_matmul_int8_inputs(M, N, K, seed=M, device="cpu")
+            out = mi.run(a.to(gpu), b.to(gpu))
+            np.testing.assert_array_equal(out.cpu().numpy()[r], oracle.matmul_int8(a.numpy()[r], b.numpy()))
+            continue
+        tdt = {"fp16": torch.float16, "fp32": torch.float32, "fp8": torch.float8_e4m3fn}[dt]
+        a, b = T.generate_matmul_fp32_fp16_fp8_inputs(M, N, K, dtype=tdt, seed=M, device="cpu")
+        out = mm.run(a.to(gpu), b.to(gpu)).cpu()
+        if dt == "fp8":
+            got = out.view(torch.uint8).numpy()[r]
+            ref = oracle.matmul_fp8(a.view(torch.uint8).numpy()[r], b.view(torch.uint8).numpy())
+            assert (got == ref).mean() > 0.995
+            g, f = oracle.e4m3_to_f32(got), oracle.e4m3_to_f32(ref)
+            step = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(f), 2.0 ** -6))) - 3)
+            assert (np.abs(g - f) <= step + 1e-12).all()
+        elif dt == "fp16":
+            ref = oracle.matmul_f16(a.numpy()[r], b.numpy()).astype(np.float32)
+            np.testing.assert_allclose(out.numpy()[r].astype(np.float32), ref, atol=2e-3, rtol=2e-3)
+        else:
+            np.testing.assert_allclose(out.numpy()[r], oracle.matmul_f32(a.numpy()[r], b.numpy()), atol=1e-4, rtol=1e-4)
+
+
+def test_plain_fp8_product_to_a_4_byte_aligned_output(gpu):
+    """tb_matmul_fp8_bt takes an output on 4 bytes: the small tiles store 8-byte
+    granules, so such an output takes the 256 x 256 tiles."""
+    M, N, K = 65, 200, 256
+    _say("plain fp8, output on 4 bytes", M, N, K)
+    a, b = T.generate_matmul_fp32_fp16_fp8_inputs(M, N, K, dtype=torch.float8_e4m3fn, seed=1, device="cpu")
+    ag, bt = a.to(gpu), b.t().contiguous().to(gpu)
+    buf = torch.zeros(M * N + 16, dtype=torch.uint8, device=gpu)
+    out = torch.zeros(M * N, dtype=torch.uint8, device=gpu)
+    for dst in (buf.data_ptr() + 4, out.data_ptr()):
+        rt.call("tb_matmul_fp8_bt", ag.data_ptr(), bt.data_ptr(), dst, M, N, K, rt.stream_handle())
+    torch.cuda.synchronize()
+    assert torch.equal(buf[4:4 + M * N], out) and int(buf[:4].sum()) == 0 and int(buf[4 + M * N:].sum()) == 0

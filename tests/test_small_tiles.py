@@ -1,4 +1,4 @@
-"""The rules that pick a W4A16 or fp8 tile (tilebench_amd/csrc/small_plan.h): the sizes
+"""The rules that pick a W4A16, fp8 or plain-product tile (tilebench_amd/csrc/small_plan.h): the sizes
 of the GPU parity tests run the tile they are listed under."""
 import os
 import shutil
@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES, FP8_TILE_IDS, FP8_TILES
+from small_tile_cases import DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES, FP8_TILE_IDS, FP8_TILES, NT_TILE_IDS, NT_TILES
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -42,3 +42,11 @@ def test_fp8_tiles_picked(tmp_path):
     args = [str(x) for _, *c in cases for x in c]
     got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
     assert [int(g) for g in got] == [FP8_TILE_IDS[c[0]] for c in cases]
+
+
+def test_plain_product_tiles_picked(tmp_path):
+    exe = _build(tmp_path)
+    cases = [(tile, M, -10 ** 9 - Kb, N) for tile, cs in NT_TILES.items() for M, N, Kb in cs]
+    args = [str(x) for _, *c in cases for x in c]
+    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
+    assert [int(g) for g in got] == [NT_TILE_IDS[c[0]] for c in cases]

@@ -36,4 +36,4 @@ def run(a: torch.Tensor, b: torch.Tensor, **kwargs):
 
 
 def get_last_config():
-    return {"kernel": "nt_gemm", "tile": "256x256"}
+    return {"kernel": "nt_gemm", "tile": "by size"}

@@ -27,14 +27,13 @@ def run(a: torch.Tensor, b: torch.Tensor, **kwargs):
 
 
 def _config(M, N, K):
-    """The kernel choice of tb_matmul_int8 (nt_gemm.hip: big_tiles, int8_splits)."""
+    """The kernel choice of tb_matmul_int8 (nt_gemm.hip: int8_splits; the tile of
+    an unsplit product is plan::pick_nt_tile's)."""
     tiles256 = -(-M // 256) * -(-N // 256)
-    if tiles256 >= 256:
-        return {"kernel": "nt_gemm<i8>", "tile": "256x256", "k_splits": 1}
-    splits = min(8, 256 // tiles256, K // 128 // 8)
+    splits = 1 if tiles256 >= 256 else min(8, 256 // tiles256, K // 128 // 8)
     if splits >= 2:
         return {"kernel": "nt_gemm<i8>", "tile": "256x256", "k_splits": splits}
-    return {"kernel": "nt_gemm<i8>", "tile": "128x128", "k_splits": 1}
+    return {"kernel": "nt_gemm<i8>", "tile": "by size", "k_splits": 1}
 
 
 _last_config = None

@@ -19,9 +19,9 @@
 // c ^ ((r ^ (r >> 3)) & 7) (conflict-free DMA writes and fragment reads).
 // The MFMA takes the B^T fragment as its first operand, so each lane ends with
 // four consecutive output columns per accumulator group and stores them
-// straight from registers.  Two tile shapes: 256 x 256 on eight wavefronts
-// (128 x 64 each) and 128 x 128 on four (64 x 64 each) for grids too small for
-// 256 x 256 tiles.  matmul_int8 at M = N = 2048 (64 tiles of 256 x 256) splits
+// straight from registers.  One 256 x 256 tile per block on eight wavefronts
+// (128 x 64 each); grids of too few such tiles run nt_small (64 x 64, 64 x 128 or
+// 128 x 128 tiles, plan::pick_nt_tile).  matmul_int8 at M = N = 2048 (64 tiles of 256 x 256) splits
 // K instead when K is deep: 128 x 128 int8 tiles need 32 KiB of operands per
 // CU per 128-byte K step, about the L2-to-CU bandwidth at the MFMA rate, where
 // 256 x 256 tiles need half that per MAC; each split writes an int32 partial
@@ -34,6 +34,7 @@
 // K' = 3K of A' = [A_hi | A_hi | A_lo] and B'^T = [B_hi^T | B_lo^T | B_hi^T],
 // accurate to about 2^-16 per product: finer than the TF32 the reference
 // allows for its fp32 matmul (10 mantissa bits) and run at the bf16 rate.
+#include "small_plan.h"
 #include "tb_common.h"
 
 #include <algorithm>
@@ -360,6 +361,191 @@ __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64, 1)
   }
 }
 
+// Small tiles for grids of too few 256 x 256 tiles: one 64 FI x 64 FJ tile per
+// block (FI, FJ = 1 or 2), four wavefronts of FI x FJ fragments, an ST-stage ring
+// of 128-byte K steps fed by DMA, as fp8_small.hip's fp8_tile: while one
+// k-substep's MFMAs run the next one's fragments are read, and one barrier per
+// step, before its last substep, hands the stage on.  Bound by LDS reads (128 x
+// 128) or, with few tiles, by the latency of a step, which the smaller tiles
+// shorten.  Same MFMA operands in the same K order as nt_gemm, so the results are
+// bit-identical to it.
+template <int KIND, int OUT, int FI, int FJ, int ST>
+struct Small {
+  static constexpr int TM = 64 * FI, TN = 64 * FJ, A_ST = TM * BK, STAGE = A_ST + TN * BK;
+  static constexpr int OSZ = OUT == OUT_E4M3 ? 1 : OUT == OUT_F16 || OUT == OUT_BF16 ? 2 : 4;
+  static constexpr int CS = TN * OSZ + 16;  // staged output row (bytes)
+  static constexpr int LDS_BYTES = ST * STAGE > TM * CS ? ST * STAGE : TM * CS;
+};
+
+template <int KIND, int OUT, int FI, int FJ, int ST>
+__global__ void __launch_bounds__(256, 1)
+    nt_small(const uint8_t* __restrict__ A, const uint8_t* __restrict__ BT, uint8_t* __restrict__ Y, int M, int N,
+             int Kb, int tiles_m) {
+  typedef Small<KIND, OUT, FI, FJ, ST> C;
+  typedef typename Acc<KIND>::type acc_t;
+  constexpr int SUB = KIND == KIND_FP8 ? 2 : 4, NFR = FI + FJ, NQ = FI * FJ;
+  extern __shared__ __attribute__((aligned(128))) uint8_t lds[];
+  // blocks go round-robin over the 8 XCDs: each takes a contiguous run of tiles, in
+  // groups of 8 tile rows (column by column inside a group), so that an XCD's L2
+  // serves neighbouring tiles
+  const int nb = gridDim.x, x = (int)blockIdx.x & 7, rem = nb & 7;
+  const int idx = x * (nb >> 3) + min(x, rem) + ((int)blockIdx.x >> 3);
+  const int tiles_n = nb / tiles_m, first = idx / (8 * tiles_n) * 8, rows = min(tiles_m - first, 8);
+  const int in_group = idx - first * tiles_n;
+  const int n0 = in_group / rows * C::TN, m0 = (first + in_group % rows) * C::TM;
+  const int t = threadIdx.x, lane = t & 63, r = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 1, wn = wave & 1;
+  const int nk = Kb / BK;
+  const i32x4 ra = make_rsrc4(A, (uint32_t)M * (uint32_t)Kb), rb = make_rsrc4(BT, (uint32_t)N * (uint32_t)Kb);
+  const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(
+      __attribute__((address_space(3))) void*)lds);
+
+  // DMA d of a step: 8 A rows per instruction for d < DA, then 8 B rows
+  constexpr int DA = 2 * FI, DB = 2 * FJ, PER = DA + DB;
+  uint32_t off[PER];
+#pragma unroll
+  for (int d = 0; d < PER; ++d) {
+    const int row = 8 * (d < DA ? DA * wave + d : DB * wave + d - DA) + (lane >> 3);
+    const int c = (lane & 7) ^ ((row ^ (row >> 3)) & 7), g = (d < DA ? m0 : n0) + row;
+    off[d] = g < (d < DA ? M : N) ? (uint32_t)g * (uint32_t)Kb + (uint32_t)c * 16u : OOB;
+  }
+  auto issue_one = [&](int k, int st, int d) __attribute__((always_inline)) {
+    const bool live = k < nk;  // past the last step: empty resources (zeros, no traffic)
+    i32x4 rs = d < DA ? ra : rb;
+    rs[2] = __builtin_amdgcn_readfirstlane(live ? rs[2] : 0);
+    const uint32_t dst = d < DA ? (uint32_t)(8 * (DA * wave + d) * BK) : (uint32_t)(C::A_ST + 8 * (DB * wave + d - DA) * BK);
+    dma16(lds0 + (uint32_t)(st * C::STAGE) + dst, off[d], rs, (uint32_t)(live ? k : 0) * BK);
+  };
+
+  // fragment f (f < FI: A rows 32 (FI wm + f) .., then B rows) of substep s: fp8
+  // chunks 4 s + 2 h and + 1 of the lane's row, the others chunk 2 s + h
+  typedef __attribute__((address_space(3))) uint8_t lds_u8;
+  typedef __attribute__((address_space(3))) const i32x4 lds_i4;
+  constexpr int HALVES = KIND == KIND_FP8 ? 2 : 1;
+  uint32_t base[NFR][HALVES];
+#pragma unroll
+  for (int f = 0; f < NFR; ++f)
+#pragma unroll
+    for (int q = 0; q < HALVES; ++q) {
+      const int row = 32 * (f < FI ? FI * wm + f : FJ * wn + f - FI) + r;
+      base[f][q] = lds0 + (uint32_t)((f < FI ? 0 : C::A_ST) + slot(row, HALVES * h + q));
+    }
+  struct Frag {
+    i32x8 v[NFR];
+  };
+  auto read_one = [&](Frag& fr, int st, int s, int f) __attribute__((always_inline)) {
+    // substep s flips address bits from 16 * 2 * HALVES on
+    const uint32_t flip = (uint32_t)(s * 32 * HALVES);
+    const i32x4 lo = *(lds_i4*)((lds_u8*)(uintptr_t)(base[f][0] ^ flip) + st * C::STAGE);
+    if constexpr (KIND == KIND_FP8) {
+      const i32x4 hi = *(lds_i4*)((lds_u8*)(uintptr_t)(base[f][HALVES - 1] ^ flip) + st * C::STAGE);
+      fr.v[f] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+      fr.v[f] = i32x8{lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0};
+    }
+  };
+
+  acc_t acc[FI][FJ];
+#pragma unroll
+  for (int i = 0; i < FI; ++i)
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) acc[i][j] = acc_t{};
+
+  constexpr int VM0 = PER * (ST - 1), VM1 = PER * (ST - 2);
+  static_assert(VM0 < 64, "vmcnt range");
+  constexpr int WAIT_PRO = (VM0 & 15) | ((VM0 >> 4) << 14) | (7 << 4) | (15 << 8);
+  constexpr int WAIT_STEP = (VM1 & 15) | ((VM1 >> 4) << 14) | (7 << 4) | (0 << 8);
+  auto barrier = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int st = 0; st < ST; ++st)
+#pragma unroll
+    for (int d = 0; d < PER; ++d) issue_one(st, st, d);
+  __builtin_amdgcn_s_waitcnt(WAIT_PRO);
+  barrier();
+  Frag fr[2];
+#pragma unroll
+  for (int f = 0; f < NFR; ++f) read_one(fr[0], 0, 0, f);
+  auto step = [&](int k, int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < SUB; ++s) {
+      const bool last = s == SUB - 1;
+      if (last) {
+        // step k + 1 landed, and every wavefront has read this stage
+        __builtin_amdgcn_s_waitcnt(WAIT_STEP);
+        barrier();
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int i = q / FJ, j = q % FJ;
+        acc[i][j] = mfma<KIND>(fr[s & 1].v[FI + j], fr[s & 1].v[i], acc[i][j]);
+#pragma unroll
+        for (int f = 0; f < NFR; ++f)
+          if (f * NQ / NFR == q) read_one(fr[(s & 1) ^ 1], last ? (st + 1) % ST : st, last ? 0 : s + 1, f);
+        if (last) {
+#pragma unroll
+          for (int d = 0; d < PER; ++d)
+            if (d * NQ / PER == q) issue_one(k + ST, st, d);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  for (int k = 0; k < nk; k += ST) {
+#pragma unroll
+    for (int st = 0; st < ST; ++st)
+      if (k + st < nk) step(k + st, st);
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  // elements 4g .. 4g + 3 of fragment (i, j): row 32 (FI wm + i) + r, columns 32 (FJ
+  // wn + j) + 8 g + 4 h ..; staged in LDS so that the stores write whole row runs
+#pragma unroll
+  for (int i = 0; i < FI; ++i)
+#pragma unroll
+    for (int j = 0; j < FJ; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        uint8_t* const p = lds + (32 * (FI * wm + i) + r) * C::CS + (32 * (FJ * wn + j) + 8 * g + 4 * h) * C::OSZ;
+        if constexpr (OUT == OUT_I32 || OUT == OUT_F32) {
+          i32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const auto x = acc[i][j][4 * g + e];  // a value: the builtin would cast a vector element's whole vector
+            v[e] = __builtin_bit_cast(int, x);
+          }
+          *reinterpret_cast<i32x4*>(p) = v;
+        } else if constexpr (OUT == OUT_F16) {
+          u32x2 v;
+          v[0] = as_u32(f16x2{(_Float16)acc[i][j][4 * g], (_Float16)acc[i][j][4 * g + 1]});
+          v[1] = as_u32(f16x2{(_Float16)acc[i][j][4 * g + 2], (_Float16)acc[i][j][4 * g + 3]});
+          *reinterpret_cast<u32x2*>(p) = v;
+        } else {  // OUT_E4M3: the bf16 value, cast once more
+          uint32_t c = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            c |= e4m3_code(__builtin_bit_cast(float, bf16_bits((float)acc[i][j][4 * g + e]) << 16)) << (8 * e);
+          *reinterpret_cast<uint32_t*>(p) = c;
+        }
+      }
+  __syncthreads();
+  constexpr int CH = OUT == OUT_E4M3 ? 8 : 16;  // store granule: N % 8 == 0 columns of one byte are 8-byte granules
+  constexpr int CPR = C::TN * C::OSZ / CH;
+  for (int q = t; q < C::TM * CPR; q += 256) {
+    const int row = q / CPR, b = q % CPR * CH;
+    if (m0 + row >= M || n0 + b / C::OSZ >= N) continue;
+    uint8_t* const dst = Y + ((int64_t)(m0 + row) * N + n0) * C::OSZ + b;
+    if constexpr (CH == 8)
+      *reinterpret_cast<u32x2*>(dst) = *reinterpret_cast<const u32x2*>(lds + row * C::CS + b);
+    else
+      *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(lds + row * C::CS + b);
+  }
+}
+
 // ------------------------------------------------------------------ preparation passes
 
 // The preparation passes move 64 x 64 element tiles through LDS with 16-byte
@@ -556,8 +742,41 @@ inline int int8_splits(int64_t M, int64_t N, int64_t K) {
   return s >= 2 ? (int)s : 1;
 }
 
-// 256 x 256 tiles when they alone fill the device, else 128 x 128.
-inline bool big_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256) >= 256; }
+template <int KIND, int OUT, int FI, int FJ, int ST>
+tb_status launch_small(const uint8_t* A, const uint8_t* BT, void* Y, int64_t M, int64_t N, int64_t Kb,
+                       hipStream_t stream, const char* what) {
+  typedef Small<KIND, OUT, FI, FJ, ST> C;
+  auto kern = &nt_small<KIND, OUT, FI, FJ, ST>;
+  constexpr size_t lds = C::LDS_BYTES;
+  if (tb_status st = reserve_lds(reinterpret_cast<const void*>(kern), lds, what)) return st;
+  const int tiles_m = (int)((M + C::TM - 1) / C::TM), tiles_n = (int)((N + C::TN - 1) / C::TN);
+  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(256), lds, stream, A, BT, reinterpret_cast<uint8_t*>(Y), (int)M,
+                     (int)N, (int)Kb, tiles_m);
+  return launch_status(what);
+}
+
+// The product on the tile plan::pick_nt_tile picks.  Ring stages: four of 64 x 64
+// (16 x 4096 x 4096 fp16 14.7 against 16.5 us with three), three otherwise, two
+// where several 128 x 128 tiles share a CU so that two blocks fit (1690 x 3432 x
+// 2176 fp16 34 against 40 us).
+template <int KIND, int OUT>
+tb_status launch_any(const uint8_t* A, const uint8_t* BT, void* Y, int64_t M, int64_t N, int64_t Kb,
+                     hipStream_t stream, const char* what) {
+  // e4m3 rows are stored in 8-byte granules by the small tiles, in 4-byte ones by nt_gemm
+  const plan::NtTile tile = OUT == OUT_E4M3 && !aligned(Y, 8) ? plan::NT_256 : plan::pick_nt_tile(M, N, Kb);
+  switch (tile) {
+    case plan::NT_64x64:
+      return launch_small<KIND, OUT, 1, 1, 4>(A, BT, Y, M, N, Kb, stream, what);
+    case plan::NT_64x128:
+      return launch_small<KIND, OUT, 1, 2, 3>(A, BT, Y, M, N, Kb, stream, what);
+    case plan::NT_128x128:
+      if (((M + 127) / 128) * ((N + 127) / 128) <= 256)
+        return launch_small<KIND, OUT, 2, 2, 3>(A, BT, Y, M, N, Kb, stream, what);
+      return launch_small<KIND, OUT, 2, 2, 2>(A, BT, Y, M, N, Kb, stream, what);
+    default:
+      return launch_nt<KIND, OUT, 256, 256, 128, 64>(A, BT, Y, nullptr, nullptr, M, N, Kb, stream, what);
+  }
+}
 
 }  // namespace ntg
 }  // namespace tb
@@ -593,11 +812,7 @@ extern "C" tb_status tb_matmul_fp8_bt(const uint8_t* a, const uint8_t* bT, uint8
   TB_CHECK_ALIGN(a, 16, "a");
   TB_CHECK_ALIGN(bT, 16, "bT");
   TB_CHECK_ALIGN(out, 4, "out");
-  if (big_tiles(M, N))
-    return launch_nt<KIND_FP8, OUT_E4M3, 256, 256, 128, 64>(a, bT, out, nullptr, nullptr, M, N, K, stream,
-                                                             "tb_matmul_fp8_bt");
-  return launch_nt<KIND_FP8, OUT_E4M3, 128, 128, 64, 64>(a, bT, out, nullptr, nullptr, M, N, K, stream,
-                                                         "tb_matmul_fp8_bt");
+  return launch_any<KIND_FP8, OUT_E4M3>(a, bT, out, M, N, K, stream, "tb_matmul_fp8_bt");
 }
 
 extern "C" tb_status tb_matmul(int dtype, const void* a, const void* b, void* out, int64_t M, int64_t N, int64_t K,
@@ -621,7 +836,6 @@ extern "C" tb_status tb_matmul(int dtype, const void* a, const void* b, void* ou
   TB_CHECK_ALIGN(out, 16, "out");
   const dim3 tgrid((unsigned)((N + 63) / 64), (unsigned)((K + 63) / 64));
   uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
-  const bool big = big_tiles(M, N);
   if (dtype == 0) {
     uint16_t* Ap = reinterpret_cast<uint16_t*>(ws);
     uint16_t* Bp = Ap + 3 * M * K;
@@ -629,22 +843,14 @@ extern "C" tb_status tb_matmul(int dtype, const void* a, const void* b, void* ou
                        reinterpret_cast<const float*>(a), Ap, (int)M, (int)K);
     hipLaunchKernelGGL(split_transpose, tgrid, dim3(256), 0, stream, reinterpret_cast<const float*>(b), Bp, (int)K,
                        (int)N);
-    if (big)
-      return launch_nt<KIND_BF16, OUT_F32, 256, 256, 128, 64>(reinterpret_cast<const uint8_t*>(Ap),
-                                                              reinterpret_cast<const uint8_t*>(Bp), out, nullptr,
-                                                              nullptr, M, N, kb, stream, "tb_matmul(fp32)");
-    return launch_nt<KIND_BF16, OUT_F32, 128, 128, 64, 64>(reinterpret_cast<const uint8_t*>(Ap),
-                                                           reinterpret_cast<const uint8_t*>(Bp), out, nullptr, nullptr,
-                                                           M, N, kb, stream, "tb_matmul(fp32)");
+    return launch_any<KIND_BF16, OUT_F32>(reinterpret_cast<const uint8_t*>(Ap), reinterpret_cast<const uint8_t*>(Bp), out,
+                                          M, N, kb, stream, "tb_matmul(fp32)");
   }
   if (dtype == 1) {
     hipLaunchKernelGGL(transpose_tile<2>, tgrid, dim3(256), 0, stream, reinterpret_cast<const uint8_t*>(b), ws,
                        (int)K, (int)N);
-    if (big)
-      return launch_nt<KIND_F16, OUT_F16, 256, 256, 128, 64>(reinterpret_cast<const uint8_t*>(a), ws, out, nullptr,
-                                                             nullptr, M, N, kb, stream, "tb_matmul(fp16)");
-    return launch_nt<KIND_F16, OUT_F16, 128, 128, 64, 64>(reinterpret_cast<const uint8_t*>(a), ws, out, nullptr,
-                                                          nullptr, M, N, kb, stream, "tb_matmul(fp16)");
+    return launch_any<KIND_F16, OUT_F16>(reinterpret_cast<const uint8_t*>(a), ws, out, M, N, kb, stream,
+                                         "tb_matmul(fp16)");
   }
   const dim3 tgrid1((unsigned)((N + TILE_B - 1) / TILE_B), (unsigned)((K + TILE_B - 1) / TILE_B));
   hipLaunchKernelGGL(transpose_tile<1>, tgrid1, dim3(256), 0, stream, reinterpret_cast<const uint8_t*>(b), ws, (int)K,
@@ -683,11 +889,6 @@ extern "C" tb_status tb_matmul_int8(const int8_t* a, const uint8_t* b, int32_t* 
                        reinterpret_cast<const i32x4*>(planes), reinterpret_cast<i32x4*>(out), n4, splits);
     return tb::launch_status("tb_matmul_int8(reduce)");
   }
-  if (big_tiles(M, N))
-    return launch_nt<KIND_I8, OUT_I32, 256, 256, 128, 64>(reinterpret_cast<const uint8_t*>(a),
-                                                          reinterpret_cast<const uint8_t*>(bt), out, nullptr, nullptr,
-                                                          M, N, K, stream, "tb_matmul_int8");
-  return launch_nt<KIND_I8, OUT_I32, 128, 128, 64, 64>(reinterpret_cast<const uint8_t*>(a),
-                                                       reinterpret_cast<const uint8_t*>(bt), out, nullptr, nullptr, M,
-                                                       N, K, stream, "tb_matmul_int8");
+  return launch_any<KIND_I8, OUT_I32>(reinterpret_cast<const uint8_t*>(a), reinterpret_cast<const uint8_t*>(bt), out, M,
+                                      N, K, stream, "tb_matmul_int8");
 }

@@ -1,4 +1,4 @@
-// Which tile a W4A16 or scaled fp8 product runs on: host-only C++ (no HIP),
+// Which tile a W4A16, scaled fp8 or plain product runs on: host-only C++ (no HIP),
 // shared with a CPU check.
 //
 // A W4A16 product's time is about its K steps times the time of one step of all its
@@ -113,6 +113,31 @@ inline Fp8Tile pick_fp8_tile(int64_t M, int64_t N, int64_t K, bool block_scaled)
   take(FP8_64x128, 3 * std::max(1.0, t64x128 / 2) + s * (0.30 * t64x128 + 0.03));
   take(FP8_64x64, 3 * std::max(1.0, t64 / 2) + s * std::max(block_scaled ? 0.25 : 0.20, 0.19 * t64));
   take(FP8_32x32, up(tiles(32, 32)) * (1.5 + (double)(std::min<int64_t>(32, M) + 32) * (double)K / 33e3));
+  return best;
+}
+
+enum NtTile { NT_256 = 0, NT_64x64, NT_64x128, NT_128x128 };
+
+// The tile of a plain product (Kb: bytes of K per operand row), by the same
+// estimate: a step of 128 bytes takes 0.2 us at 64 x 64, 0.31 at 64 x 128, 0.4 -
+// 0.6 at 128 x 128 and 1.35 - 1.95 at 256 x 256 (fp16; the other types within a
+// fifth).  Measured fp16 products alone, us: 16 x 4096 x 4096 14.7 (64 x 64;
+// 256 x 256 86), 512 x 4096 x 4096 23.4 (64 x 128; 93), 2048 x 2048 x 4096 39 (128 x
+// 128; 95), 2601 x 1648 x 2432 30 (128 x 128; 58), 3362 x 2504 x 5248 120 (256 x
+// 256; 128 x 128 128), 4096 x 4096 x 4096 129 (256 x 256; 128 x 128 135).
+inline NtTile pick_nt_tile(int64_t M, int64_t N, int64_t Kb) {
+  const double s = (double)Kb / 128;
+  auto tiles = [&](int64_t tm, int64_t tn) { return (double)((M + tm - 1) / tm * ((N + tn - 1) / tn)) / 256.0; };
+  auto up = [](double v) { return (double)(int64_t)(v + 0.999999); };
+  const double big = tiles(256, 256), t128 = tiles(128, 128), t64x128 = up(tiles(64, 128)), t64 = up(tiles(64, 64));
+  double c = 3 * std::max(1.0, big) + s * (big <= 1 ? 1.35 + 0.2 * big + std::max(0.0, big - 0.6) : 1.95 * big);
+  NtTile best = NT_256;
+  auto take = [&](NtTile t, double cost) {
+    if (cost < c) best = t, c = cost;
+  };
+  take(NT_128x128, 3 * std::max(1.0, t128 / 2) + s * (t128 <= 1 ? 0.4 + 0.2 * t128 : t128 <= 2 ? 0.9 : std::max(1.6, 0.53 * t128)));
+  take(NT_64x128, 3 * std::max(1.0, t64x128 / 2) + s * (0.30 * t64x128 + 0.03));
+  take(NT_64x64, 3 * std::max(1.0, t64 / 2) + s * std::max(0.2, 0.19 * t64));
   return best;
 }
 
