@@ -1,13 +1,13 @@
 """GPU parity of the small W4A16 tiles (w4a16_small.hip): every tile of the
 dense, grouped, gate/up and down products against the CPU oracle, and bit for bit
-against the 256-row tiles on the same rows; and of the small-tile scaled
+against the 256-row tiles on the same rows; of the decode's slab widths and splits; and of the small-tile scaled
 fp8 (fp8_small.hip) and plain products (nt_gemm.hip) against the oracle."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
-from small_tile_cases import DENSE_TILES, EXPERT_TILES, FP8_TILES, NT_TILES
+from small_tile_cases import DECODE_PLANS, DENSE_TILES, EXPERT_TILES, FP8_TILES, NT_TILES
 from tilebench_amd import runtime as rt
 from tilebench_amd.data import tensors as T
 
@@ -130,6 +130,24 @@ def test_dense_rows_do_not_depend_on_the_tile(gpu, M):
     torch.cuda.synchronize()
     assert torch.equal(small.view(torch.int16), big[:M].view(torch.int16))
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("cols,splits", list(DECODE_PLANS))
+def test_decode_plans_match_oracle(gpu, cols, splits):
+    """Each slab width and split of the decode at 1, 5 and 16 rows, twice in a row
+    (the arrival counters are back at zero) with equal bits."""
+    from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
+
+    for N, K in DECODE_PLANS[cols, splits]:
+        for M in (1, 5, 16):
+            _say("decode", cols, splits, M, N, K)
+            A, p, s, z, G = T.generate_w4a16_gemm_inputs(M, K, N, 64, seed=N + K + M, device="cpu")
+            d = [t.to(gpu) for t in (A, p, s, z)]
+            Y, Y2 = impl_hip.run(*d, G), impl_hip.run(*d, G)
+            torch.cuda.synchronize()
+            assert torch.equal(Y.view(torch.int16), Y2.view(torch.int16))
+            ref = oracle.w4a16_gemm(A.numpy(), p.numpy(), s.numpy(), z.numpy(), G)
+            np.testing.assert_allclose(Y.cpu().numpy().astype(np.float32), ref.astype(np.float32), atol=1e-2, rtol=1e-2)
 
 
 @pytest.mark.parametrize("tile", list(FP8_TILES))

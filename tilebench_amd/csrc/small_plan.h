@@ -141,5 +141,38 @@ inline NtTile pick_nt_tile(int64_t M, int64_t N, int64_t Kb) {
   return best;
 }
 
+constexpr int DEC_WAVES = 8, DEC_UNIT = 32, DEC_MAX_SPLITS = 16;
+struct DecodePlan {
+  int cols;       // columns of a slab, 128 or 256
+  int64_t slabs;
+  int splits;     // blocks that share a slab's K
+};
+
+// Slab width and K splits of the W4A16 decode kernel by an estimate of its time
+// (us at M = 16): a wavefront takes its 32-row units one after the other, 0.75
+// each at 128 columns and 1.45 at 256; a split costs an exchange of partials (1.5
+// or 3) that grows with the blocks taking part (0.55 or 0.6 each); and 128-column
+// slabs, which read half lines, lose 0.11 per MB of weights.  Measured, 128 / 256
+// columns at their best splits: K 4096, N 4096 7.8 / 11.4; K 4096, N 11008 11.4 /
+// 12.5; K 4096, N 12288 13.5 / 13.2; K 8192, N 28672 43.1 / 32.6.  Splits at 128
+// columns, K 4096, N 4096: 1 13.1, 2 9.7, 4 7.8, 8 8.5; K 1024, N 12288: 1 6.0, 2 6.7.
+// A split grid never has more blocks than CUs.
+inline DecodePlan pick_decode(int64_t N, int64_t K, int cus) {
+  const int64_t units = K / DEC_UNIT;
+  DecodePlan best{256, (N + 255) / 256, 1};
+  double c = -1;
+  for (int cols = 128; cols <= 256; cols += 128) {
+    const bool wide = cols == 256;
+    const int64_t slabs = (N + cols - 1) / cols;
+    for (int s = 1; s <= DEC_MAX_SPLITS && (s == 1 || (slabs * s <= cus && (int64_t)s * DEC_WAVES <= units)); ++s) {
+      const int64_t rounds = (slabs * s + cus - 1) / cus, chain = (units + (int64_t)s * DEC_WAVES - 1) / (s * DEC_WAVES);
+      double cost = (double)(rounds * chain) * (wide ? 1.45 : 0.75) + (wide ? 0.0 : 0.11e-6 * 0.5 * (double)N * (double)K);
+      if (s > 1) cost += wide ? 3 + 0.6 * s : 1.5 + 0.55 * s;
+      if (c < 0 || cost < c) best = DecodePlan{cols, slabs, s}, c = cost;
+    }
+  }
+  return best;
+}
+
 }  // namespace plan
 }  // namespace tb

@@ -75,21 +75,24 @@ struct Tile {
 };
 
 // ---------------------------------------------------------------------------
-// Decode kernel (M <= 16, HBM-bound on the weights).  A block of eight
-// wavefronts owns a 256-column slab and one of S contiguous K ranges, and the
-// grid never holds more blocks than the device has CUs (one block fills a CU),
-// so every block starts at once.  Each wavefront streams its own contiguous
+// Decode kernel (M <= 16, HBM-bound on the weights when they are large, else on
+// the latency of a block's chain of loads and of the partials' exchange).  A
+// block of eight wavefronts owns a slab of 256 columns, or 128 where those give
+// the shorter chain (plan::pick_decode), and one of S contiguous K ranges; where
+// K is split the grid never holds more blocks than the device has CUs, so every
+// block starts at once.  Each wavefront streams its own contiguous
 // run of 32-row units, the next unit's loads issued as soon as a unit has been
 // consumed (one unit in flight per wavefront: the chip's loads then arrive
 // early enough for compute to overlap them; deeper prefetch measured slower).
 // Per unit a lane loads an 8 x 16 int4 block (eight 8-byte row loads; 16 lanes
-// side by side cover a full 128-byte line of a row) and its A fragment; a
+// side by side cover a full 128-byte line of a row; 8 x 8 and half a line at 128
+// columns) and its A fragment; a
 // group's scales and zero-points are loaded once, at the group's first unit.
 // All are buffer loads whose offsets are out of range (zeros, no traffic) where
 // a row, column or unit does not exist, so no load sits behind a branch and
 // the compiler's wait before a unit covers only that unit.  The MFMAs
 // (v_mfma_f32_16x16x32_f16, A rows >= M zero; fragment f holds columns
-// 16c + f, c = lane % 16) take the codes themselves as c0 + q (c0 = 1024 for
+// 16c + f, or 8c + f, c = lane % 16) take the codes themselves as c0 + q (c0 = 1024 for
 // even columns, 64 for odd ones), built from the packed bytes by one byte
 // permute per two rows and an and-or per nibble (under one VALU instruction
 // per weight, against 2.4 for dequantising each weight first); the scale and
@@ -100,13 +103,17 @@ struct Tile {
 // them, as the reference dequantisation does); the difference stays far below
 // the 1e-2 tolerance.  The eight wave partials are summed in LDS in a fixed
 // order, so results are reproducible bit for bit.
+// Measured at M = 16, us, 256-column slabs alone -> now: K 4096, N 4096 14.4 ->
+// 7.8; K 4096, N 11008 12.8 -> 11.8; K 11008, N 4096 16.0 -> 12.1; K 1024, N 12288
+// 10.1 -> 6.1; K 8192, N 28672 (256 columns) 32.6, 3.6 TB/s.
 // Across the S blocks of a slab the reduction is a serial split-K: each block
 // writes its fp32 partial through to the device-coherent level, then bumps the
 // slab's arrival counter; the block that arrives last reads the S partials
 // (all loads in flight at once), adds them in slot order (deterministic),
 // writes fp16 Y and puts the counter back to zero, so the workspace is ready
 // for the next call without any clearing.
-constexpr int DEC_COLS = 256, DEC_THREADS = 512, DEC_WAVES = 8, DEC_UNIT = 32, DEC_MAX_SPLITS = 16;
+constexpr int DEC_THREADS = 512, DEC_WAVES = plan::DEC_WAVES, DEC_UNIT = plan::DEC_UNIT;
+constexpr int DEC_MAX_SPLITS = plan::DEC_MAX_SPLITS;
 constexpr int AUX_SC1 = 16;  // buffer cache policy: coherent across the XCDs
 // Workspace layout, the same for every shape so that calls of different shapes
 // can share one buffer: [DEC_MAX_SLABS int32 arrival counters][fp32 partials].
@@ -116,29 +123,38 @@ constexpr int64_t DEC_COUNTER_BYTES = DEC_MAX_SLABS * 4;
 
 typedef float f32x4d __attribute__((ext_vector_type(4)));
 
+template <int WORDS>
 struct DecUnit {
-  u32x2 w[8];  // rows kg*8 + r, columns 16c .. 16c + 15
-  u32x4 a;     // A row lane % 16, k = kg*8 .. +7
+  uint32_t w[8][WORDS];  // rows kg*8 + r, the lane's 8 WORDS columns
+  u32x4 a;               // A row lane % 16, k = kg*8 .. +7
 };
+template <int WORDS>
 struct DecGroup {
-  u32x4 s0, s1;  // scales of the group, columns 16c .. 16c + 15
-  uint32_t z0, z1;  // zero-points of the group, columns 16c .. 16c + 15
+  u32x4 s[WORDS];  // scales of the group, the lane's columns
+  uint32_t z[WORDS];
 };
 
-template <bool TAIL>
-__global__ void __launch_bounds__(DEC_THREADS)
+template <int WORDS, bool TAIL>
+__global__ void __launch_bounds__(DEC_THREADS, 2)
     w4a16_decode(const _Float16* __restrict__ A, const uint8_t* __restrict__ W, const _Float16* __restrict__ S,
                  const uint8_t* __restrict__ Z, _Float16* __restrict__ Y, float* __restrict__ partials,
                  int* __restrict__ counters, int M, int N, int K, int group, int splits) {
-  __shared__ float part[DEC_WAVES][16 * DEC_COLS];  // 128 KiB: one partial per wavefront
+  constexpr int DEC_COLS = 128 * WORDS, CPL = 8 * WORDS;  // columns of the slab, of a lane
+  __shared__ float part[DEC_WAVES][16 * DEC_COLS];  // one partial per wavefront
   __shared__ int last_flag;
-  const int slab = blockIdx.x / splits, split = blockIdx.x % splits;
+  // 128-column slabs come in pairs that share their rows' 128-byte lines: both
+  // halves of a pair run on one XCD (block ids 8 apart), next to each other in time
+  int item = blockIdx.x;
+  if (WORDS == 1) item = (item >> 4) * 8 + (item & 7);
+  const int slab = WORDS == 1 ? item / splits * 2 + (((int)blockIdx.x >> 3) & 1) : item / splits;
+  const int split = item % splits;
+  if (WORDS == 1 && slab * DEC_COLS >= N) return;  // the grid is rounded up to pairs on 8 XCDs
   const int n0 = slab * DEC_COLS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, kg = lane >> 4;
-  const int n = n0 + c * 16;
+  const int n = n0 + c * CPL;
   const bool col_ok = n < N;               // at least columns n .. n+7 exist (N % 8 == 0)
-  const bool col_full = n + 16 <= N;       // all 16 columns exist
+  const bool col_full = n + CPL <= N;      // all of the lane's columns exist
   const int units = K / DEC_UNIT;
   const int u_begin = (int)((int64_t)units * split / splits), u_end = (int)((int64_t)units * (split + 1) / splits);
   const int bu = u_end - u_begin;
@@ -157,36 +173,44 @@ __global__ void __launch_bounds__(DEC_THREADS)
   const uint32_t w_off = col_full ? (uint32_t)(kg * 8) * half_n + (uint32_t)(n >> 1) : OOB;
   const uint32_t w_tail = (TAIL && col_ok && !col_full) ? (uint32_t)(kg * 8) * half_n + (uint32_t)(n >> 1) : OOB;
   const uint32_t a_off = arow < M ? ((uint32_t)arow * (uint32_t)K + (uint32_t)(kg * 8)) * 2u : OOB;
-  const uint32_t s_off0 = col_ok ? (uint32_t)n * 2u : OOB, s_off1 = col_full ? (uint32_t)(n + 8) * 2u : OOB;
-  const uint32_t z_off0 = col_ok ? (uint32_t)(n >> 1) : OOB, z_off1 = col_full ? (uint32_t)(n >> 1) + 4u : OOB;
-  constexpr int NT = 2;  // nontemporal: the weights are read once
+  const uint32_t s_off[2] = {col_ok ? (uint32_t)n * 2u : OOB, col_full ? (uint32_t)(n + 8) * 2u : OOB};
+  const uint32_t z_off[2] = {col_ok ? (uint32_t)(n >> 1) : OOB, col_full ? (uint32_t)(n >> 1) + 4u : OOB};
+  // nontemporal where the weights are large and read once; not where the other half of
+  // the line is about to be read on the same XCD (172 blocks at M = 1 11.7 us, nontemporal 12.3)
+  constexpr int NT = WORDS == 1 ? 0 : 2;
 
-  f32x4d acc[16];
+  f32x4d acc[CPL];
 #pragma unroll
-  for (int f = 0; f < 16; ++f) acc[f] = f32x4d{};
+  for (int f = 0; f < CPL; ++f) acc[f] = f32x4d{};
 
   // A unit past the wavefront's range is still issued, with an out-of-range
   // offset (no memory traffic, zeros): the loop has no branch around a load.
-  auto load_unit = [&](DecUnit& d, int u) {
+  auto load_unit = [&](DecUnit<WORDS>& d, int u) {
     const bool live = u < w_end;
     const uint32_t kw = live ? (uint32_t)(u * DEC_UNIT) * half_n : OOB;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      d.w[r] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, w_off + (uint32_t)r * half_n, kw, NT));
-      if (TAIL) {
-        const uint32_t t = __builtin_amdgcn_raw_buffer_load_b32(rw, w_tail + (uint32_t)r * half_n, kw, NT);
-        d.w[r] = col_full ? d.w[r] : u32x2{t, 0u};
+      if constexpr (WORDS == 1) {
+        d.w[r][0] = __builtin_amdgcn_raw_buffer_load_b32(rw, w_off + (uint32_t)r * half_n, kw, NT);
+      } else {
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, w_off + (uint32_t)r * half_n, kw, NT));
+        d.w[r][0] = v[0], d.w[r][1] = v[1];
+        if (TAIL) {
+          const uint32_t t = __builtin_amdgcn_raw_buffer_load_b32(rw, w_tail + (uint32_t)r * half_n, kw, NT);
+          d.w[r][0] = col_full ? v[0] : t, d.w[r][1] = col_full ? v[1] : 0u;
+        }
       }
     }
     d.a = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off, live ? (uint32_t)(u * DEC_UNIT) * 2u : OOB, 0);
   };
   // A group's scales and zero-points, needed only by its fold.
-  auto load_group = [&](DecGroup& d, int g) {
+  auto load_group = [&](DecGroup<WORDS>& d, int g) {
     const uint32_t ks = (uint32_t)g * (uint32_t)N * 2u, kz = (uint32_t)g * half_n;
-    d.s0 = __builtin_amdgcn_raw_buffer_load_b128(rs, s_off0, ks, 0);
-    d.s1 = __builtin_amdgcn_raw_buffer_load_b128(rs, s_off1, ks, 0);
-    d.z0 = __builtin_amdgcn_raw_buffer_load_b32(rz, z_off0, kz, 0);
-    d.z1 = __builtin_amdgcn_raw_buffer_load_b32(rz, z_off1, kz, 0);
+#pragma unroll
+    for (int h = 0; h < WORDS; ++h) {
+      d.s[h] = __builtin_amdgcn_raw_buffer_load_b128(rs, s_off[h], ks, 0);
+      d.z[h] = __builtin_amdgcn_raw_buffer_load_b32(rz, z_off[h], kz, 0);
+    }
   };
   // One unit's MFMAs on the raw codes: B fragment f holds column 16c + f as
   // c0 + q (exact in fp16) for the lane's 8 rows, built straight from the
@@ -198,13 +222,13 @@ __global__ void __launch_bounds__(DEC_THREADS)
   // scale and zero-point are applied once per group to the fp32 sums (fold
   // below); a ninth-row MFMA against ones accumulates the A row sums it needs.
   const h8 ones = __builtin_bit_cast(h8, u32x4{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u});
-  auto mma_unit = [&](const DecUnit& d, f32x4d (&tmp)[16], f32x4d& asum, auto first) {
+  auto mma_unit = [&](const DecUnit<WORDS>& d, f32x4d (&tmp)[CPL], f32x4d& asum, auto first) {
     constexpr bool FIRST = decltype(first)::value;
     const f32x4d zero{};
     const h8 af = __builtin_bit_cast(h8, d.a);
     asum = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, ones, FIRST ? zero : asum, 0, 0, 0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < WORDS; ++h) {
       u32x4 col[8];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -227,12 +251,12 @@ __global__ void __launch_bounds__(DEC_THREADS)
   // Fold of one group: sum_k a (q - z) s = s (sum_k a (c0 + q) - (c0 + z) sum_k a),
   // c0 = 1024 for even columns f and 64 for odd ones, in fp32, for the rows
   // e < M only (rows past M are never stored).
-  auto fold = [&](const f32x4d (&tmp)[16], const f32x4d& asum, const DecGroup& gp) {
+  auto fold = [&](const f32x4d (&tmp)[CPL], const f32x4d& asum, const DecGroup<WORDS>& gp) {
 #pragma unroll
-    for (int f = 0; f < 16; ++f) {
-      const u32x4 sv = f < 8 ? gp.s0 : gp.s1;
+    for (int f = 0; f < CPL; ++f) {
+      const u32x4 sv = gp.s[f / 8];
       const float sf = (float)__builtin_bit_cast(_Float16, (uint16_t)(sv[(f % 8) / 2] >> (16 * (f & 1))));
-      const float zf = (float)((f & 1 ? 64u : 1024u) + (((f < 8 ? gp.z0 : gp.z1) >> (4 * (f % 8))) & 15u));
+      const float zf = (float)((f & 1 ? 64u : 1024u) + ((gp.z[f / 8] >> (4 * (f % 8))) & 15u));
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (e < M) acc[f][e] = __builtin_fmaf(sf, __builtin_fmaf(-zf, asum[e], tmp[f][e]), acc[f][e]);
@@ -246,14 +270,14 @@ __global__ void __launch_bounds__(DEC_THREADS)
   // wavefront: double buffering measured slower, the weights' stream being
   // the limit).
   const int upg = group / DEC_UNIT;
-  DecUnit buf;
+  DecUnit<WORDS> buf;
   load_unit(buf, w_begin);
   int u = w_begin;
   while (u < w_end) {
     const int gend = min(w_end, (u / upg + 1) * upg);
-    DecGroup gp;
+    DecGroup<WORDS> gp;
     load_group(gp, u / upg);
-    f32x4d tmp[16], asum;
+    f32x4d tmp[CPL], asum;
     mma_unit(buf, tmp, asum, std::true_type{});
     load_unit(buf, ++u);
     for (; u < gend; ++u) {
@@ -263,14 +287,19 @@ __global__ void __launch_bounds__(DEC_THREADS)
     fold(tmp, asum, gp);
   }
 
-  // Accumulator f, element e: row 4 * (lane / 16) + e, column 16c + f.
+  // Accumulator f, element e: row 4 * (lane / 16) + e, column CPL c + f.  A row's
+  // 16-byte chunks are ordered by f / 4, then c, so that the 16 lanes of a write
+  // meet 16 different bank groups (ordered by column they met four).
 #pragma unroll
-  for (int f = 0; f < 16; ++f)
+  for (int e = 0; e < 4; ++e)
+    if (4 * kg + e < M)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) part[wave][(4 * kg + e) * DEC_COLS + c * 16 + f] = acc[f][e];
+      for (int f = 0; f < CPL; f += 4)
+        *reinterpret_cast<f32x4d*>(&part[wave][(4 * kg + e) * DEC_COLS + (f * 4 + c) * 4]) =
+            f32x4d{acc[f][e], acc[f + 1][e], acc[f + 2][e], acc[f + 3][e]};
   __syncthreads();
   // Fixed-order sum of the eight wave partials; thread t owns the float4 chunks
-  // t and t + 512 of the 16 x 256 tile.
+  // t and t + 512 of the tile (the first only at 128 columns).
   const int ncols = min(DEC_COLS, N - n0);
   constexpr int CH = 16 * DEC_COLS / 4 / DEC_THREADS;
   f32x4d red[CH];
@@ -284,7 +313,7 @@ __global__ void __launch_bounds__(DEC_THREADS)
   }
   auto store_y = [&](int q, f32x4d v) {
     const int i = (threadIdx.x + q * DEC_THREADS) * 4;
-    const int m = i / DEC_COLS, cc = i % DEC_COLS;
+    const int m = i / DEC_COLS, ch = i % DEC_COLS / 4, cc = ch % 16 * CPL + ch / 16 * 4;
     if (m < M && cc < ncols) {  // ncols % 8 == 0, so a chunk is all in or all out
       u32x2 h;
       h[0] = as_u32(f16x2{(_Float16)v[0], (_Float16)v[1]});
@@ -310,12 +339,12 @@ __global__ void __launch_bounds__(DEC_THREADS)
   // that reads splits - 1 then loads the partials with sc1, which reads them
   // from that same coherence point, never from a stale line of its XCD's L2.
   // A release / acquire pair on the counter would add an L2 write-back
-  // (buffer_wbl2) to every block and an invalidate to the last one; measured
-  // on the box, that made the M = 1 decode about 4 us slower.
+  // (buffer_wbl2) to every block and an invalidate to the last one, which made
+  // the M = 1 decode about 4 us slower.
   const rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(partials, 0, 0x7FFFFFFF, (int)RSRC_DW3);
   auto poff = [&](int s2, int q) -> uint32_t {
     const int i = (threadIdx.x + q * DEC_THREADS) * 4;
-    const int m = i / DEC_COLS, cc = i % DEC_COLS;
+    const int m = i / DEC_COLS, ch = i % DEC_COLS / 4, cc = ch % 16 * CPL + ch / 16 * 4;
     return (m < M && cc < ncols) ? (uint32_t)((((int64_t)s2 * M + m) * N + n0 + cc) * 4) : OOB;
   };
 #pragma unroll
@@ -359,15 +388,7 @@ inline int device_cus() {
   return cache[dev];
 }
 
-// One block per CU: slabs x splits never exceeds the CU count.
-inline int decode_splits(int N, int K) {
-  const int slabs = (N + DEC_COLS - 1) / DEC_COLS;
-  const int units = K / DEC_UNIT;
-  int s = device_cus() / slabs;
-  s = std::min(s, DEC_MAX_SPLITS);
-  s = std::min(s, units / DEC_WAVES);
-  return std::max(s, 1);
-}
+inline plan::DecodePlan decode_plan(int64_t N, int64_t K) { return plan::pick_decode(N, K, device_cus()); }
 
 // ---------------------------------------------------------------- dense prefill
 namespace p8 {
@@ -1306,8 +1327,7 @@ extern "C" tb_status tb_w4a16_workspace_size(int64_t M, int64_t N, int64_t K, in
   TB_CHECK_ARG(M > 0 && N > 0 && K > 0 && group > 0, "tb_w4a16_workspace_size: sizes must be positive");
   *bytes = 0;
   if (M <= 16 && K % DEC_UNIT == 0) {
-    const int64_t slabs = (N + DEC_COLS - 1) / DEC_COLS;
-    const int splits = decode_splits((int)N, (int)K);
+    const int splits = decode_plan(N, K).splits;
     if (splits > 1) *bytes = DEC_COUNTER_BYTES + (int64_t)splits * M * N * 4;
   }
   return TB_OK;
@@ -1339,9 +1359,8 @@ static tb_status check_dense_args(const char* fn, const uint16_t* A, const uint8
   TB_CHECK_ALIGN(zeros, 4, "zeros");
   TB_CHECK_ALIGN(Y, 2, "Y");
   if (M <= 16) {
-    const int64_t slabs = (N + DEC_COLS - 1) / DEC_COLS;
-    const int splits = decode_splits((int)N, (int)K);
-    TB_CHECK_ARG(splits == 1 || (slabs <= DEC_MAX_SLABS && (int64_t)splits * M * N * 4 < (1ll << 31)),
+    const plan::DecodePlan p = decode_plan(N, K);
+    TB_CHECK_ARG(p.splits == 1 || (p.slabs <= DEC_MAX_SLABS && (int64_t)p.splits * M * N * 4 < (1ll << 31)),
                  "%s: N=%lld is too wide for the decode kernel", fn, (long long)N);
   }
   return TB_OK;
@@ -1361,19 +1380,22 @@ static tb_status launch_dense(const char* fn, const uint16_t* A, const uint8_t* 
                               const uint8_t* zeros, uint16_t* Y, int64_t M, int64_t N, int64_t K, int64_t group,
                               void* workspace, hipStream_t stream) {
   if (M <= 16) {
-    const int64_t slabs = (N + DEC_COLS - 1) / DEC_COLS;
-    const int splits = decode_splits((int)N, (int)K);
+    const plan::DecodePlan p = decode_plan(N, K);
     int* counters = reinterpret_cast<int*>(workspace);
     float* partials =
-        splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + DEC_COUNTER_BYTES) : nullptr;
-    if (N % 16 == 0)
-      hipLaunchKernelGGL(w4a16_decode<false>, dim3((unsigned)(slabs * splits)), dim3(DEC_THREADS), 0, stream,
+        p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + DEC_COUNTER_BYTES) : nullptr;
+    auto launch = [&](auto kern, int64_t blocks) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(DEC_THREADS), 0, stream,
                          reinterpret_cast<const _Float16*>(A), W, reinterpret_cast<const _Float16*>(scales), zeros,
-                         reinterpret_cast<_Float16*>(Y), partials, counters, (int)M, (int)N, (int)K, (int)group, splits);
+                         reinterpret_cast<_Float16*>(Y), partials, counters, (int)M, (int)N, (int)K, (int)group,
+                         p.splits);
+    };
+    if (p.cols == 128)
+      launch(w4a16_decode<1, false>, ((p.slabs + 1) / 2 * p.splits + 7) / 8 * 16);
+    else if (N % 16 == 0)
+      launch(w4a16_decode<2, false>, p.slabs * p.splits);
     else
-      hipLaunchKernelGGL(w4a16_decode<true>, dim3((unsigned)(slabs * splits)), dim3(DEC_THREADS), 0, stream,
-                         reinterpret_cast<const _Float16*>(A), W, reinterpret_cast<const _Float16*>(scales), zeros,
-                         reinterpret_cast<_Float16*>(Y), partials, counters, (int)M, (int)N, (int)K, (int)group, splits);
+      launch(w4a16_decode<2, true>, p.slabs * p.splits);
     return tb::launch_status(fn);
   }
   const auto tile = tb::plan::pick_dense_tile(M, N);
@@ -1398,7 +1420,7 @@ static tb_status launch_dense(const char* fn, const uint16_t* A, const uint8_t* 
 // at M <= 16 on a 256-CU device: slabs x splits never exceeds the CU count, so
 // the partials hold at most 256 blocks x 16 rows x 256 columns of fp32
 // (4 MiB), behind the 16 KiB of counters.
-constexpr int64_t NOALLOC_SCRATCH_BYTES = DEC_COUNTER_BYTES + 256ll * 16 * DEC_COLS * 4;
+constexpr int64_t NOALLOC_SCRATCH_BYTES = DEC_COUNTER_BYTES + 256ll * 16 * 256 * 4;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 __global__ void __launch_bounds__(256) clear_counters(int* __restrict__ c, int n) {
