@@ -153,21 +153,24 @@ __global__ void __launch_bounds__(64 * KS, KS / 4 > 0 ? KS / 4 : 1)
 // c ^ ((r ^ (r >> 3)) & 7)).  While a 64-byte substep's MFMAs run, the next one's
 // fragments are read; the barrier sits between the two substeps of a step, when
 // the step's stage has been read by every wavefront and takes the DMAs of the
-// step ST later.  Bound by LDS: at 128 x 128, 64 KiB of fragment reads and 32 KiB
+// step ST later.  KG = 2 runs a second such group of wavefronts, with a ring of its
+// own, on every other step, and adds the two sums.  Bound by LDS: at 128 x 128, 64 KiB of fragment reads and 32 KiB
 // of DMA writes per step against 512 cycles of MFMAs.
 constexpr int MAXKB = 512;
 constexpr uint32_t RSRC_DW3 = 0x00020000u;
 
-template <int FI, int FJ, int ST, bool BLK>
+template <int FI, int FJ, int ST, bool BLK, int KG>
 struct Tile {
   static constexpr int TM = 64 * FI, TN = 64 * FJ;
   static constexpr int A_ST = TM * STEP, STAGE = A_ST + TN * STEP;  // A rows, then W rows
   static constexpr int SA_OFF = ST * STAGE;                         // BLK: the stages' activation scales
   static constexpr int PAD_OFF = SA_OFF + (BLK ? ST * TM * 4 : 0);  // the idle wavefronts' scale DMA lands here
-  static constexpr int SW_OFF = PAD_OFF + (BLK ? 256 : 0);          // BLK: the tile's weight scales, K / 128 floats
-  static constexpr int LDS_BYTES = SW_OFF + (BLK ? MAXKB * 4 : 0);
+  static constexpr int SW_OFF = PAD_OFF + (BLK ? 256 : 0);          // BLK, after the groups: weight scales, K / 128 floats
+  static constexpr int GROUP = SW_OFF;                              // one K group's part
+  static constexpr int LDS_BYTES = KG * GROUP + (BLK ? MAXKB * 4 : 0);
   static constexpr int C_STRIDE = TN + 8;  // bf16 per staged row (16-byte pad)
   static_assert(LDS_BYTES <= 160 * 1024 && TM * C_STRIDE * 2 <= ST * STAGE, "LDS budget");
+  static_assert(KG == 1 || TM * TN * 4 <= GROUP, "room for the other group's sums");
 };
 
 __device__ __forceinline__ i32x4 rsrc4(const void* p, uint32_t bytes) {
@@ -197,21 +200,24 @@ __device__ __forceinline__ void dma4(uint32_t lds_addr, uint32_t voff, const i32
                : "memory", "m0");
 }
 
-template <int FI, int FJ, int ST, bool BLK>
-__global__ void __launch_bounds__(256, 1)
+template <int FI, int FJ, int ST, bool BLK, int KG>
+__global__ void __launch_bounds__(256 * KG, 1)
     fp8_tile(const uint8_t* __restrict__ Aq, const uint8_t* __restrict__ WqT, const float* __restrict__ sa,
                 const float* __restrict__ sw, uint16_t* __restrict__ Y, int M, int N, int K, int tiles_m) {
-  typedef Tile<FI, FJ, ST, BLK> C;
+  typedef Tile<FI, FJ, ST, BLK, KG> C;
   extern __shared__ __attribute__((aligned(128))) uint8_t lds[];
   const int idx = xcd_run(blockIdx.x, gridDim.x);
   const int n0 = idx / tiles_m * C::TN, m0 = idx % tiles_m * C::TM;
   const int t = threadIdx.x, lane = t & 63, r = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 1, wn = wave & 1;
-  const int nk = K / STEP;
+  const int wave8 = __builtin_amdgcn_readfirstlane(t >> 6), wave = wave8 & 3, grp = wave8 >> 2;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int nk = K / STEP, ni = (nk + KG - 1) / KG;  // steps in all, of a group (its step i is step KG i + grp)
   const i32x4 ra = rsrc4(Aq, (uint32_t)M * (uint32_t)K), rw = rsrc4(WqT, (uint32_t)N * (uint32_t)K);
   const i32x4 rsa = rsrc4(sa, BLK ? (uint32_t)nk * (uint32_t)M * 4u : 0u);
-  const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(
+  const uint32_t lds_base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(
       __attribute__((address_space(3))) void*)lds);
+  const uint32_t lds0 = lds_base + (uint32_t)(grp * C::GROUP);  // the group's part
+  const uint8_t* const part = lds + grp * C::GROUP;
   auto live_rsrc = [](bool live, i32x4 v) __attribute__((always_inline)) {
     v[2] = __builtin_amdgcn_readfirstlane(live ? v[2] : 0);
     return v;
@@ -229,7 +235,8 @@ __global__ void __launch_bounds__(256, 1)
     off[d] = g < (d < DA ? M : N) ? (uint32_t)g * (uint32_t)K + (uint32_t)c * 16u : BUF_OOB;
   }
   if (BLK && wave < FI && m0 + 64 * wave + lane < M) s_off = (uint32_t)(m0 + 64 * wave + lane) * 4u;
-  auto issue_one = [&](int k, int st, int d) __attribute__((always_inline)) {
+  auto issue_one = [&](int i, int st, int d) __attribute__((always_inline)) {
+    const int k = KG * i + grp;
     const bool live = k < nk;  // past the last step: empty resources (zeros, no traffic)
     const uint32_t dst = lds0 + (uint32_t)(st * C::STAGE);
     if (d < DA)
@@ -245,8 +252,8 @@ __global__ void __launch_bounds__(256, 1)
     // the tile's weight scales sw[n0 / 128, 0 .. nk - 1], 64 per DMA (first in
     // the queue: landed before step 0's data)
     const i32x4 rsw = rsrc4(sw + (int64_t)(n0 / 128) * nk, (uint32_t)nk * 4u);
-    for (int q = wave; q < (nk + 63) / 64; q += 4)
-      dma4(lds0 + (uint32_t)(C::SW_OFF + q * 256), q * 64 + lane < nk ? (uint32_t)(q * 64 + lane) * 4u : BUF_OOB, rsw, 0u);
+    for (int q = wave8; q < (nk + 63) / 64; q += 4 * KG)
+      dma4(lds_base + (uint32_t)(KG * C::GROUP + q * 256), q * 64 + lane < nk ? (uint32_t)(q * 64 + lane) * 4u : BUF_OOB, rsw, 0u);
   }
 
   // fragment f (f < FI: A rows 32 (FI wm + f) .., then W rows 32 (FJ wn + f - FI) ..)
@@ -277,7 +284,7 @@ __global__ void __launch_bounds__(256, 1)
 #pragma unroll
     for (int j = 0; j < FJ; ++j) acc[i][j] = p[i][j] = f32x16{};
   float s_cur[FI] = {};
-  const float* const lsw = reinterpret_cast<const float*>(lds + C::SW_OFF);
+  const float* const lsw = reinterpret_cast<const float*>(lds + KG * C::GROUP);
   auto fold = [&](int i, int j) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][j][e] = __builtin_fmaf(p[i][j][e], s_cur[i], acc[i][j][e]);
@@ -303,14 +310,15 @@ __global__ void __launch_bounds__(256, 1)
   for (int f = 0; f < NFR; ++f) read_one(f0, 0, 0, f);
 
   constexpr int NQ = FI * FJ;  // MFMAs per substep
-  auto step = [&](int k, int st) __attribute__((always_inline)) {
+  auto step = [&](int i0, int st) __attribute__((always_inline)) {
     // substep 0; the stage's substep 1 read beside its MFMAs
     float s_new[FI] = {};
     if constexpr (BLK) {
-      const float b = lsw[k];
+      const int k = KG * i0 + grp;
+      const float b = KG == 1 || k < nk ? lsw[k] : 0.f;
 #pragma unroll
       for (int i = 0; i < FI; ++i)
-        s_new[i] = *reinterpret_cast<const float*>(lds + C::SA_OFF + st * C::TM * 4 + (32 * (FI * wm + i) + r) * 4) * b;
+        s_new[i] = *reinterpret_cast<const float*>(part + C::SA_OFF + st * C::TM * 4 + (32 * (FI * wm + i) + r) * 4) * b;
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -343,14 +351,14 @@ __global__ void __launch_bounds__(256, 1)
         if (f * NQ / NFR == q) read_one(f0, (st + 1) % ST, 0, f);
 #pragma unroll
       for (int e = 0; e < PER; ++e)
-        if (e * NQ / PER == q) issue_one(k + ST, st, e);
+        if (e * NQ / PER == q) issue_one(i0 + ST, st, e);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  for (int k = 0; k < nk; k += ST) {
+  for (int i = 0; i < ni; i += ST) {
 #pragma unroll
     for (int st = 0; st < ST; ++st)
-      if (k + st < nk) step(k + st, st);
+      if (i + st < ni) step(i + st, st);
   }
   if constexpr (BLK) {
 #pragma unroll
@@ -358,12 +366,33 @@ __global__ void __launch_bounds__(256, 1)
   }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
+  if constexpr (KG == 2) {  // group 0 adds group 1's sums, left in group 1's part
+    f32x4* const sums = reinterpret_cast<f32x4*>(lds + C::GROUP) + wave * (NQ * 4 * 64) + lane;
+#pragma unroll
+    for (int q = 0; q < NQ * 4; ++q) {
+      f32x16& a = acc[q / 4 / FJ][q / 4 % FJ];
+      const int g = q % 4;
+      if (grp == 1) sums[q * 64] = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NQ * 4; ++q) {
+      f32x16& a = acc[q / 4 / FJ][q / 4 % FJ];
+      const int g = q % 4;
+      if (grp == 0) {
+        const f32x4 v = sums[q * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[4 * g + e] += v[e];
+      }
+    }
+  }
 
   // element 4g + e of fragment (i, j): row 32 (FI wm + i) + r, column 32 (FJ wn + j)
   // + 8 g + 4 h + e; staged in LDS so that the stores write whole row runs
   uint16_t* const ct = reinterpret_cast<uint16_t*>(lds);
 #pragma unroll
   for (int i = 0; i < FI; ++i) {
+    if (grp != 0) break;
     const int row = 32 * (FI * wm + i) + r;
     const float s = !BLK && m0 + row < M ? sa[m0 + row] : 1.f;
 #pragma unroll
@@ -384,7 +413,7 @@ __global__ void __launch_bounds__(256, 1)
       }
   }
   __syncthreads();
-  for (int q = t; q < C::TM * (C::TN / 8); q += 256) {
+  for (int q = t; q < C::TM * (C::TN / 8); q += 256 * KG) {
     const int row = q / (C::TN / 8), ch = q % (C::TN / 8) * 8;
     if (m0 + row < M && n0 + ch < N)
       *reinterpret_cast<u32x4*>(Y + (int64_t)(m0 + row) * N + n0 + ch) =
@@ -402,34 +431,40 @@ tb_status launch_skinny(const char* fn, const Fp8Args& a, hipStream_t stream) {
   return tb::launch_status(fn);
 }
 
-template <int FI, int FJ, int ST, bool BLK>
+template <int FI, int FJ, int ST, bool BLK, int KG = 1>
 tb_status launch_tile(const char* fn, const Fp8Args& a, hipStream_t stream) {
-  typedef Tile<FI, FJ, ST, BLK> C;
-  auto kern = &fp8_tile<FI, FJ, ST, BLK>;
+  typedef Tile<FI, FJ, ST, BLK, KG> C;
+  auto kern = &fp8_tile<FI, FJ, ST, BLK, KG>;
   constexpr size_t lds = C::LDS_BYTES;
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(kern), lds, fn)) return st;
   const int64_t tiles_m = (a.M + C::TM - 1) / C::TM, tiles_n = (a.N + C::TN - 1) / C::TN;
   TB_CHECK_ARG(tiles_m * tiles_n < (1ll << 31), "%s: problem too large", fn);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), lds, stream, a.Aq, a.WqT, a.sa, a.sw, a.Y,
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256 * KG), lds, stream, a.Aq, a.WqT, a.sa, a.sw, a.Y,
                      a.M, a.N, a.K, (int)tiles_m);
   return tb::launch_status(fn);
 }
 
 // Ring stages: as deep as pays while one block runs per CU (64 x 64: four, 15.4
-// against 18.9 us with three at 64 x 8192 x 8192; with block scales the FMAs bound
-// it and three are as good); two where several 128 x 128 tiles share a CU, so that
-// two blocks fit (1024 x 8192 x 8192 60 against 70 us with three).
+// against 18.9 us with three at 64 x 8192 x 8192; 64 x 128: four, 14.0 against 15.0
+// at 512 x 4096 x 4096); two or three where several tiles share a CU, so that two
+// blocks fit (128 x 128: 1024 x 8192 x 8192 60 us with two, 70 with three).  With
+// block scales, one block per CU and one wavefront per SIMD, the scale FMAs wait for
+// the MFMAs; two K groups fill each other's waits (200 x 2112 x 7168 17.3 -> 13.8 us,
+// 128 x 8192 x 8192 20.6 -> 16.2, 300 x 5000 x 4096 14.4 -> 13.6; row scales: no gain).
 template <bool BLK>
 tb_status launch(const char* fn, plan::Fp8Tile tile, const Fp8Args& a, hipStream_t stream) {
+  auto tiles = [&](int64_t tm, int64_t tn) { return (a.M + tm - 1) / tm * ((a.N + tn - 1) / tn); };
   switch (tile) {
     case plan::FP8_32x32:
       return launch_skinny<BLK>(fn, a, stream);
     case plan::FP8_64x64:
+      if (BLK && tiles(64, 64) <= 256) return launch_tile<1, 1, 3, BLK, BLK ? 2 : 1>(fn, a, stream);
       return launch_tile<1, 1, BLK ? 3 : 4, BLK>(fn, a, stream);
     case plan::FP8_64x128:
+      if (tiles(64, 128) <= 256) return launch_tile<1, 2, BLK ? 3 : 4, BLK, BLK ? 2 : 1>(fn, a, stream);
       return launch_tile<1, 2, 3, BLK>(fn, a, stream);
     default:
-      if ((int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128) <= 256) return launch_tile<2, 2, 3, BLK>(fn, a, stream);
+      if (tiles(128, 128) <= 256) return launch_tile<2, 2, 3, BLK>(fn, a, stream);
       return launch_tile<2, 2, 2, BLK>(fn, a, stream);
   }
 }

@@ -84,15 +84,15 @@ enum Fp8Tile { FP8_256 = 0, FP8_32x32, FP8_64x64, FP8_64x128, FP8_128x128 };
 // The tile of a scaled fp8 product, by estimated time in us (s: steps of 128
 // bytes of K, x: tiles per CU; measured with s = 8 - 64).  32 x 32 blocks are
 // bound by their CU's loads, 1.5 us + (rows of A and W) x K / 33 KB per us, and
-// run in rounds of 256; a step of the LDS tiles takes 0.2 us at 64 x 64 (block
-// scales 0.25), 0.31 at 64 x 128, 0.36 - 0.5 at 128 x 128 (0.42 - 0.57), and tiles
+// run in rounds of 256; a step of the LDS tiles takes 0.2 us at 64 x 64, 0.31
+// at 64 x 128 (block scales 0.34), 0.36 - 0.5 at 128 x 128 (0.42 - 0.57), and tiles
 // that share a CU share its LDS.  A step of 256 x 256 tiles takes 0.9 us on a few
 // CUs and 1.55 us on all (1.45 and 1.9).
 // Measured, these tiles against 256 x 256 (us): 1 x 8192 x 8192 12 / 65 (32 x 32),
-// 64 x 8192 x 8192 15 / 66, 200 x 2112 x 7168 13 / 60 and 17 / 88 (64 x 64), 256 x
+// 64 x 8192 x 8192 15 / 66, 200 x 2112 x 7168 13 / 60 and 14 / 88 (64 x 64), 256 x
 // 8192 x 8192 25 / 69 (64 x 128), 512 x 8192 x 8192 35 / 69, 1024 x 4096 x 4096 23 /
-// 40, 1024 x 8192 x 8192 60 / 76 (128 x 128); 1348 x 7168 x 4224 56 / 46: the
-// 256 x 256 tiles stay.
+// 40, 1024 x 8192 x 8192 60 / 76 (128 x 128); 1348 x 7168 x 4224 56 / 46,
+// block scales 4096 x 2112 x 7168 98 (64 x 128) / 92: the 256 x 256 tiles stay.
 inline Fp8Tile pick_fp8_tile(int64_t M, int64_t N, int64_t K, bool block_scaled) {
   const double s = (double)K / 128;
   auto tiles = [&](int64_t tm, int64_t tn) { return (double)((M + tm - 1) / tm * ((N + tn - 1) / tn)) / 256.0; };
@@ -110,8 +110,8 @@ inline Fp8Tile pick_fp8_tile(int64_t M, int64_t N, int64_t K, bool block_scaled)
   else
     take(FP8_128x128, up(t128 / 2) * (3 + s * (block_scaled ? 1.04 : 0.95)));
   const double t64x128 = up(tiles(64, 128)), t64 = up(tiles(64, 64));
-  take(FP8_64x128, 3 * std::max(1.0, t64x128 / 2) + s * (0.30 * t64x128 + 0.03));
-  take(FP8_64x64, 3 * std::max(1.0, t64 / 2) + s * std::max(block_scaled ? 0.25 : 0.20, 0.19 * t64));
+  take(FP8_64x128, 3 * std::max(1.0, t64x128 / 2) + s * (block_scaled ? 0.34 * t64x128 : 0.30 * t64x128 + 0.03));
+  take(FP8_64x64, 3 * std::max(1.0, t64 / 2) + s * std::max(0.20, 0.19 * t64));
   take(FP8_32x32, up(tiles(32, 32)) * (1.5 + (double)(std::min<int64_t>(32, M) + 32) * (double)K / 33e3));
   return best;
 }
