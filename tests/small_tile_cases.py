@@ -54,5 +54,5 @@ DECODE_PLANS = {
     (128, 4): [(1408, 4096), (4096, 4096), (5000, 3072)],
     (128, 8): [(4096, 11008)],
     (256, 1): [(32776, 1024)],
-    (256, 4): [(12288, 4096), (12296, 4096)],
+    (256, 5): [(12288, 4096), (12296, 4096)],
 }

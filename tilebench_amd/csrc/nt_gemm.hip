@@ -20,8 +20,8 @@
 // The MFMA takes the B^T fragment as its first operand, so each lane ends with
 // four consecutive output columns per accumulator group and stores them
 // straight from registers.  One 256 x 256 tile per block on eight wavefronts
-// (128 x 64 each); grids of too few such tiles run nt_small (64 x 64, 64 x 128 or
-// 128 x 128 tiles, plan::pick_nt_tile).  matmul_int8 at M = N = 2048 (64 tiles of 256 x 256) splits
+// (128 x 64 each); grids of too few such tiles run 64 x 64, 64 x 128 or 128 x 128
+// tiles on four (plan::pick_nt_tile).  matmul_int8 at M = N = 2048 (64 tiles of 256 x 256) splits
 // K instead when K is deep: 128 x 128 int8 tiles need 32 KiB of operands per
 // CU per 128-byte K step, about the L2-to-CU bandwidth at the MFMA rate, where
 // 256 x 256 tiles need half that per MAC; each split writes an int32 partial
@@ -377,10 +377,13 @@ struct Small {
   static constexpr int LDS_BYTES = ST * STAGE > TM * CS ? ST * STAGE : TM * CS;
 };
 
-template <int KIND, int OUT, int FI, int FJ, int ST>
+// An overload of nt_gemm: wave tiles of WM = 32 FI rows, ST stages.
+template <int KIND, int OUT, int TM, int TN, int WM, int ST>
 __global__ void __launch_bounds__(256, 1)
-    nt_small(const uint8_t* __restrict__ A, const uint8_t* __restrict__ BT, uint8_t* __restrict__ Y, int M, int N,
+    nt_gemm(const uint8_t* __restrict__ A, const uint8_t* __restrict__ BT, uint8_t* __restrict__ Y, int M, int N,
              int Kb, int tiles_m) {
+  constexpr int FI = TM / 64, FJ = TN / 64;
+  static_assert(WM == 32 * FI, "two wavefronts side by side in each direction");
   typedef Small<KIND, OUT, FI, FJ, ST> C;
   typedef typename Acc<KIND>::type acc_t;
   constexpr int SUB = KIND == KIND_FP8 ? 2 : 4, NFR = FI + FJ, NQ = FI * FJ;
@@ -710,7 +713,8 @@ __global__ void __launch_bounds__(256) split_transpose(const float* __restrict__
 template <int KIND, int OUT, int BM, int BN, int WM, int WN>
 tb_status launch_nt(const uint8_t* A, const uint8_t* BT, void* Y, const float* sa, const float* sw, int64_t M,
                     int64_t N, int64_t Kb, hipStream_t stream, const char* what, int splits = 1) {
-  auto kern = &nt_gemm<KIND, OUT, BM, BN, WM, WN>;
+  typedef void (*Kernel)(const uint8_t*, const uint8_t*, void*, const float*, const float*, int, int, int, int, int, int);
+  const Kernel kern = &nt_gemm<KIND, OUT, BM, BN, WM, WN>;
   constexpr size_t lds = (size_t)2 * (BM + BN) * BK;
   if (tb_status st = reserve_lds(reinterpret_cast<const void*>(kern), lds, what)) return st;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
@@ -746,7 +750,8 @@ template <int KIND, int OUT, int FI, int FJ, int ST>
 tb_status launch_small(const uint8_t* A, const uint8_t* BT, void* Y, int64_t M, int64_t N, int64_t Kb,
                        hipStream_t stream, const char* what) {
   typedef Small<KIND, OUT, FI, FJ, ST> C;
-  auto kern = &nt_small<KIND, OUT, FI, FJ, ST>;
+  typedef void (*Kernel)(const uint8_t*, const uint8_t*, uint8_t*, int, int, int, int);
+  const Kernel kern = &nt_gemm<KIND, OUT, C::TM, C::TN, 32 * FI, ST>;
   constexpr size_t lds = C::LDS_BYTES;
   if (tb_status st = reserve_lds(reinterpret_cast<const void*>(kern), lds, what)) return st;
   const int tiles_m = (int)((M + C::TM - 1) / C::TM), tiles_n = (int)((N + C::TN - 1) / C::TN);

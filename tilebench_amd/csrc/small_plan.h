@@ -150,24 +150,27 @@ struct DecodePlan {
 
 // Slab width and K splits of the W4A16 decode kernel by an estimate of its time
 // (us at M = 16): a wavefront takes its 32-row units one after the other, 0.75
-// each at 128 columns and 1.45 at 256; a split costs an exchange of partials (1.5
-// or 3) that grows with the blocks taking part (0.55 or 0.6 each); and 128-column
-// slabs, which read half lines, lose 0.11 per MB of weights.  Measured, 128 / 256
-// columns at their best splits: K 4096, N 4096 7.8 / 11.4; K 4096, N 11008 11.4 /
-// 12.5; K 4096, N 12288 13.5 / 13.2; K 8192, N 28672 43.1 / 32.6.  Splits at 128
+// each at 128 columns and 1.45 at 256 (there a CU's stream binds: the mean share
+// counts, not the longest; K 4096, N 12288 from cold 14.1 on 192 CUs, 13.4 on 240); a
+// split costs an exchange of partials (1.5 or 3.6) that grows with the blocks taking
+// part (0.55 or 0.6 each); and 128-column slabs, which read half lines, lose 0.11 per
+// MB of weights.  Measured, 128 / 256 columns at their best splits: K 4096, N 4096
+// 7.8 / 11.4; K 4096, N 11008 11.4 / 12.5; K 4096, N 12288 13.5 / 13.2; K 8192, N
+// 28672 43.1 / 32.6.  Splits at 128
 // columns, K 4096, N 4096: 1 13.1, 2 9.7, 4 7.8, 8 8.5; K 1024, N 12288: 1 6.0, 2 6.7.
 // A split grid never has more blocks than CUs.
 inline DecodePlan pick_decode(int64_t N, int64_t K, int cus) {
   const int64_t units = K / DEC_UNIT;
-  DecodePlan best{256, (N + 255) / 256, 1};
+  DecodePlan best{128, (N + 127) / 128, 1};
   double c = -1;
-  for (int cols = 128; cols <= 256; cols += 128) {
+  for (int cols = 128; cols <= (N <= 128 ? 128 : 256); cols += 128) {  // the wide slab needs 16 columns
     const bool wide = cols == 256;
     const int64_t slabs = (N + cols - 1) / cols;
     for (int s = 1; s <= DEC_MAX_SPLITS && (s == 1 || (slabs * s <= cus && (int64_t)s * DEC_WAVES <= units)); ++s) {
-      const int64_t rounds = (slabs * s + cus - 1) / cus, chain = (units + (int64_t)s * DEC_WAVES - 1) / (s * DEC_WAVES);
-      double cost = (double)(rounds * chain) * (wide ? 1.45 : 0.75) + (wide ? 0.0 : 0.11e-6 * 0.5 * (double)N * (double)K);
-      if (s > 1) cost += wide ? 3 + 0.6 * s : 1.5 + 0.55 * s;
+      const double rounds = (double)((slabs * s + cus - 1) / cus), share = (double)units / (s * DEC_WAVES);
+      double cost = wide ? rounds * std::max(1.0, share) * 1.45
+                         : rounds * (double)(int64_t)(share + 0.999999) * 0.75 + 0.055e-6 * (double)N * (double)K;
+      if (s > 1) cost += wide ? 3.6 + 0.6 * s : 1.5 + 0.55 * s;
       if (c < 0 || cost < c) best = DecodePlan{cols, slabs, s}, c = cost;
     }
   }

@@ -134,11 +134,13 @@ struct DecGroup {
   uint32_t z[WORDS];
 };
 
-template <int WORDS, bool TAIL>
+// WIDE: 256-column slabs, 16 columns to a lane; else 128 and 8.
+template <bool WIDE>
 __global__ void __launch_bounds__(DEC_THREADS, 2)
     w4a16_decode(const _Float16* __restrict__ A, const uint8_t* __restrict__ W, const _Float16* __restrict__ S,
                  const uint8_t* __restrict__ Z, _Float16* __restrict__ Y, float* __restrict__ partials,
                  int* __restrict__ counters, int M, int N, int K, int group, int splits) {
+  constexpr int WORDS = WIDE ? 2 : 1;  // of a lane in a row
   constexpr int DEC_COLS = 128 * WORDS, CPL = 8 * WORDS;  // columns of the slab, of a lane
   __shared__ float part[DEC_WAVES][16 * DEC_COLS];  // one partial per wavefront
   __shared__ int last_flag;
@@ -152,9 +154,11 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
   const int n0 = slab * DEC_COLS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, kg = lane >> 4;
-  const int n = n0 + c * CPL;
-  const bool col_ok = n < N;               // at least columns n .. n+7 exist (N % 8 == 0)
-  const bool col_full = n + CPL <= N;      // all of the lane's columns exist
+  // A lane of 16 columns whose last 8 do not exist (N % 16 == 8) also takes the 8 before
+  // its first, its neighbour's, so that every load is whole; it stages only its own.
+  const bool col_ok = n0 + c * CPL < N;  // at least 8 columns exist (N % 8 == 0)
+  const int extra = WIDE && col_ok && n0 + c * CPL + CPL > N ? 8 : 0;
+  const int n = n0 + c * CPL - extra;    // >= 0: N = 8 takes 128-column slabs
   const int units = K / DEC_UNIT;
   const int u_begin = (int)((int64_t)units * split / splits), u_end = (int)((int64_t)units * (split + 1) / splits);
   const int bu = u_end - u_begin;
@@ -170,11 +174,10 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
   const rsrc_t ra = make_rsrc(A, (uint32_t)M * (uint32_t)K * 2u);
   const rsrc_t rs = make_rsrc(S, (uint32_t)(K / group) * (uint32_t)N * 2u);
   const rsrc_t rz = make_rsrc(Z, (uint32_t)(K / group) * half_n);
-  const uint32_t w_off = col_full ? (uint32_t)(kg * 8) * half_n + (uint32_t)(n >> 1) : OOB;
-  const uint32_t w_tail = (TAIL && col_ok && !col_full) ? (uint32_t)(kg * 8) * half_n + (uint32_t)(n >> 1) : OOB;
+  const uint32_t w_off = col_ok ? (uint32_t)(kg * 8) * half_n + (uint32_t)(n >> 1) : OOB;
   const uint32_t a_off = arow < M ? ((uint32_t)arow * (uint32_t)K + (uint32_t)(kg * 8)) * 2u : OOB;
-  const uint32_t s_off[2] = {col_ok ? (uint32_t)n * 2u : OOB, col_full ? (uint32_t)(n + 8) * 2u : OOB};
-  const uint32_t z_off[2] = {col_ok ? (uint32_t)(n >> 1) : OOB, col_full ? (uint32_t)(n >> 1) + 4u : OOB};
+  const uint32_t s_off[2] = {col_ok ? (uint32_t)n * 2u : OOB, col_ok ? (uint32_t)(n + 8) * 2u : OOB};
+  const uint32_t z_off[2] = {col_ok ? (uint32_t)(n >> 1) : OOB, col_ok ? (uint32_t)(n >> 1) + 4u : OOB};
   // nontemporal where the weights are large and read once; not where the other half of
   // the line is about to be read on the same XCD (172 blocks at M = 1 11.7 us, nontemporal 12.3)
   constexpr int NT = WORDS == 1 ? 0 : 2;
@@ -195,10 +198,6 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
       } else {
         const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, w_off + (uint32_t)r * half_n, kw, NT));
         d.w[r][0] = v[0], d.w[r][1] = v[1];
-        if (TAIL) {
-          const uint32_t t = __builtin_amdgcn_raw_buffer_load_b32(rw, w_tail + (uint32_t)r * half_n, kw, NT);
-          d.w[r][0] = col_full ? v[0] : t, d.w[r][1] = col_full ? v[1] : 0u;
-        }
       }
     }
     d.a = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off, live ? (uint32_t)(u * DEC_UNIT) * 2u : OOB, 0);
@@ -295,8 +294,9 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
     if (4 * kg + e < M)
 #pragma unroll
       for (int f = 0; f < CPL; f += 4)
-        *reinterpret_cast<f32x4d*>(&part[wave][(4 * kg + e) * DEC_COLS + (f * 4 + c) * 4]) =
-            f32x4d{acc[f][e], acc[f + 1][e], acc[f + 2][e], acc[f + 3][e]};
+        if (f >= extra)
+          *reinterpret_cast<f32x4d*>(&part[wave][(4 * kg + e) * DEC_COLS + ((f - extra) * 4 + c) * 4]) =
+              f32x4d{acc[f][e], acc[f + 1][e], acc[f + 2][e], acc[f + 3][e]};
   __syncthreads();
   // Fixed-order sum of the eight wave partials; thread t owns the float4 chunks
   // t and t + 512 of the tile (the first only at 128 columns).
@@ -1391,11 +1391,9 @@ static tb_status launch_dense(const char* fn, const uint16_t* A, const uint8_t* 
                          p.splits);
     };
     if (p.cols == 128)
-      launch(w4a16_decode<1, false>, ((p.slabs + 1) / 2 * p.splits + 7) / 8 * 16);
-    else if (N % 16 == 0)
-      launch(w4a16_decode<2, false>, p.slabs * p.splits);
+      launch(w4a16_decode<false>, ((p.slabs + 1) / 2 * p.splits + 7) / 8 * 16);
     else
-      launch(w4a16_decode<2, true>, p.slabs * p.splits);
+      launch(w4a16_decode<true>, p.slabs * p.splits);
     return tb::launch_status(fn);
   }
   const auto tile = tb::plan::pick_dense_tile(M, N);
