@@ -43,7 +43,7 @@ def run(X, logits, W13, S13, Z13, W2, S2, Z2, topk: int, group13: int, group2: i
             W2.data_ptr(), S2.data_ptr(), Z2.data_ptr(), out.data_ptr(), T, E, topk, H, I, group13, group2,
             rt.ptr(ws), need, rt.stream_handle(X.device))
     _last_config = {"kernels": ["gating", "moe_align", "moe_gate_up", "moe_down", "moe_combine"],
-                    "BM": 256, "BN_gate_up": 128, "BN_down": 256, "workspace_bytes": need}
+                    "BM": "by size", "BN_gate_up": "by size", "BN_down": "by size", "workspace_bytes": need}
     return out
 
 

@@ -76,7 +76,7 @@ def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torc
             M, N, K, group, rt.ptr(ws), need.value, stream)
     _last_config = ({"kernel": "w4a16_decode", "layout": "rows", "cols_per_block": "by size",
                      "workspace_bytes": need.value}
-                    if M <= 16 else {"kernel": "w4a16_prefill", "layout": "rows", "BM": 256, "BN": 256, "BK": 64})
+                    if M <= 16 else {"kernel": "w4a16_prefill", "layout": "rows", "BM": "by size", "BN": "by size", "BK": 64})
     return Y
 
 
