@@ -222,3 +222,14 @@ def test_plain_fp8_product_to_a_4_byte_aligned_output(gpu):
         rt.call("tb_matmul_fp8_bt", ag.data_ptr(), bt.data_ptr(), dst, M, N, K, rt.stream_handle())
     torch.cuda.synchronize()
     assert torch.equal(buf[4:4 + M * N], out) and int(buf[:4].sum()) == 0 and int(buf[4 + M * N:].sum()) == 0
+
+
+@pytest.mark.parametrize("form", ["none", "cuda", "cuda:0", "index", "device"])
+def test_stream_handle_takes_every_form_of_a_device(gpu, form):
+    device = {"none": None, "index": 0, "device": torch.device("cuda", 0)}.get(form, form)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert rt.stream_handle(device) == side.cuda_stream
+    assert rt.stream_handle(device) == torch.cuda.current_stream().cuda_stream
+    with pytest.raises(ValueError):
+        rt.stream_handle(torch.device("cpu", 0))
