@@ -132,6 +132,23 @@ def test_dense_rows_do_not_depend_on_the_tile(gpu, M):
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("M", [17, 31, 32])
+@pytest.mark.parametrize("K,N", [(64, 8), (704, 1000), (2048, 4096)])  # N % 32 != 0 and == 0
+def test_dense_32_row_tile(gpu, M, K, N):
+    """Up to 32 rows: the oracle's values, and the bits of the same rows on a 64-row tile."""
+    from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
+
+    _say("dense 32 rows", M, K, N)
+    A, p, s, z, G = T.generate_w4a16_gemm_inputs(33, K, N, 64, seed=M + N, device="cpu")
+    d = [t.to(gpu) for t in (A, p, s, z)]
+    big = impl_hip.run(*d, G)
+    small = impl_hip.run(d[0][:M].contiguous(), *d[1:], G)
+    torch.cuda.synchronize()
+    assert torch.equal(small.view(torch.int16), big[:M].view(torch.int16))
+    ref = oracle.w4a16_gemm(A.numpy()[:M], p.numpy(), s.numpy(), z.numpy(), G)
+    np.testing.assert_allclose(small.cpu().numpy().astype(np.float32), ref.astype(np.float32), atol=1e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("cols,splits", list(DECODE_PLANS))
 def test_decode_plans_match_oracle(gpu, cols, splits):
     """Each slab width and split of the decode at 1, 5 and 16 rows, twice in a row

@@ -56,7 +56,8 @@ enum DenseTile { DENSE_256 = 0, DENSE_64x64_K4, DENSE_64x128, DENSE_64x256, DENS
 // K step, measured at K = 4096 and 11008 on 43 - 1376 tiles).  Up to 64 rows
 // 64-column tiles of four K groups put a product on every CU that has columns
 // for it: 48 rows x 11008 columns 15 us against 25 (64 x 128), 30 (64 x 256)
-// and 62 (256 x 256).  128 x 11008 (K = 4096): 64 x 128 25 us, 64 x 256 31, 128
+// and 62 (256 x 256); up to 32 rows the launch halves its rows (12.5 at 32 rows,
+// 13.9 on 64).  128 x 11008 (K = 4096): 64 x 128 25 us, 64 x 256 31, 128
 // x 256 42, 256 x 256 63; 512 x 11008: 61 / 59 / 52 / 71; 1024 x 11008: 116 /
 // 101 / 106 / 95; 500 x 4096 (K = 11008): 65 / 78 / 106 / 160.
 inline DenseTile pick_dense_tile(int64_t M, int64_t N) {

@@ -27,7 +27,7 @@
 // dequantisation to fp16, the same v_mfma_f32_32x32x16_f16 operands in the same
 // K order per output element, the same epilogue roundings; results are
 // bit-identical to them, so neither the choice of tile nor the call that uses
-// it shows in an output.  Only the dense product of at most 64 rows (S64x64k4)
+// it shows in an output.  Only the dense product of at most 64 rows (S32x64k4, S64x64k4)
 // splits K, over four groups of wavefronts of one block whose fp32 sums are
 // added through LDS in group order: reproducible, but not the unsplit order.
 // No workspace is needed.
@@ -74,6 +74,7 @@ struct Shape {
 typedef Shape<1, 2, true, 1, 3> S32x128;
 typedef Shape<1, 4, false, 1, 3> S32x256;
 typedef Shape<2, 4, false, 1, 3> S64x256;
+typedef Shape<1, 1, true, 1, 3, 4> S32x64k4;
 typedef Shape<2, 1, true, 1, 3, 4> S64x64k4;
 typedef Shape<2, 2, true, 1, 4> S64x128;
 typedef Shape<4, 4, false, 1, 3> S128x256;
@@ -571,6 +572,13 @@ tb_status launch_dense_small(const char* fn, plan::DenseTile tile, const DenseAr
   const bool wide = tb::aligned(a.W, 16) && a.N % 32 == 0;
   switch (tile) {
     case plan::DENSE_64x64_K4:
+      // Up to 32 rows half of a 64-row tile's MFMAs, A DMAs and A reads are padding
+      // that the CU's LDS and load paths carry (deeper rings or other K group
+      // counts gained nothing).  The same K groups in the same order: the bits are those of
+      // the 64-row tile.  Kernel, us, 64 -> 32 rows: 32 x 11008 (K 4096) 13.9 -> 12.5, 24 x
+      // 4096 (K 11008) 33.2 -> 29.0, 20 x 12288 (K 1024) 7.3 -> 6.3.
+      if (a.M <= 32)
+        return wide ? launch_dense_shape<S32x64k4, true>(fn, a, stream) : launch_dense_shape<S32x64k4, false>(fn, a, stream);
       return wide ? launch_dense_shape<S64x64k4, true>(fn, a, stream) : launch_dense_shape<S64x64k4, false>(fn, a, stream);
     case plan::DENSE_64x128:
       return wide ? launch_dense_shape<S64x128, true>(fn, a, stream) : launch_dense_shape<S64x128, false>(fn, a, stream);
