@@ -328,6 +328,41 @@ tb_status tb_matmul_fp8_bt(const uint8_t* a, const uint8_t* bT, uint8_t* out, in
 tb_status tb_matmul_workspace_size(int dtype, int64_t M, int64_t N, int64_t K, int64_t* bytes);
 
 /*
+ * The kernel and tile that a GEMM entry point launches for these sizes on the
+ * current device (host code: nothing is launched; operands aligned to 16
+ * bytes).  `kernel` is a static string.  A block computes tile_rows x tile_cols
+ * of the product on `wavefronts` wavefronts; within it k_groups groups of them
+ * take parts of K, and k_splits blocks share one tile's K.  Gate/up (N = 2 I): its
+ * tile_cols columns of W13 are tile_cols / 2 activation columns.
+ *   op                     M                N      experts
+ *   TB_OP_W4A16            rows             N      ignored
+ *   TB_OP_W4A16_GROUPED    R                N      E
+ *   TB_OP_MOE_GATE_UP      tokens * topk    2 I    E
+ *   TB_OP_MOE_DOWN         tokens * topk    H      E
+ *   TB_OP_FP8_SCALED, _FP8_BLOCK, _MATMUL_F32, _F16, _FP8, _INT8: ignored
+ * Replaces: the get_last_config() of the reference's tuned operators
+ * (matmul_fp32_fp16_fp8/impl_triton.py:124), which reports the configuration
+ * that ran.
+ */
+enum {
+  TB_OP_W4A16 = 0,
+  TB_OP_W4A16_GROUPED = 1,
+  TB_OP_MOE_GATE_UP = 2,
+  TB_OP_MOE_DOWN = 3,
+  TB_OP_FP8_SCALED = 4,
+  TB_OP_FP8_BLOCK = 5,
+  TB_OP_MATMUL_F32 = 6,
+  TB_OP_MATMUL_F16 = 7,
+  TB_OP_MATMUL_FP8 = 8,
+  TB_OP_MATMUL_INT8 = 9
+};
+typedef struct {
+  const char* kernel;
+  int32_t tile_rows, tile_cols, wavefronts, k_groups, k_splits;
+} tb_tile;
+tb_status tb_gemm_tile(int op, int64_t M, int64_t N, int64_t K, int64_t experts, tb_tile* tile);
+
+/*
  * Fill `bytes` bytes of `buf` with a 32-bit pattern using a plain store
  * kernel (cache-allocating stores: nontemporal ones would leave the MALL's
  * contents in place).  Used to evict the L2 and the 256 MiB MALL between

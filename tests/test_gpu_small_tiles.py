@@ -250,3 +250,51 @@ def test_stream_handle_takes_every_form_of_a_device(gpu, form):
     assert rt.stream_handle(device) == torch.cuda.current_stream().cuda_stream
     with pytest.raises(ValueError):
         rt.stream_handle(torch.device("cpu", 0))
+
+
+@pytest.mark.parametrize("op,case", [
+    ("w4a16_gemm", dict(M=16, K=4096, N=4096)), ("w4a16_gemm", dict(M=20, K=256, N=1024)),
+    ("w4a16_gemm", dict(M=48, K=256, N=1024)), ("w4a16_gemm", dict(M=300, K=512, N=512)),
+    ("w4a16_gemm", dict(M=1024, K=128, N=11008)),
+    ("fp8_scaled_gemm", dict(M=16, N=8192, K=896)), ("fp8_scaled_gemm", dict(M=300, N=5000, K=384)),
+    ("fp8_block_scaled_gemm", dict(M=200, N=2112, K=1152)), ("fp8_block_scaled_gemm", dict(M=1024, N=8200, K=1152)),
+    ("moe_w4a16_grouped_gemm", dict(tokens=64, topk=2, experts=8, K=256, N=264)),
+    ("fused_moe_w4a16", dict(tokens=24, experts=8, topk=2, H=256, I=128)),
+    ("matmul_fp32_fp16_fp8", dict(M=513, N=2056, K=320, dtype="fp16")),
+    ("matmul_int8", dict(M=100, N=1000, K=640, dtype="int8")),
+], ids=lambda x: x if isinstance(x, str) else None)
+def test_config_names_what_was_launched(gpu, op, case):
+    """get_last_config() after a call against the kernels the profiler saw: the
+    name, and the tile from the template arguments."""
+    import importlib
+    import re
+
+    from tilebench_amd.profiling import probe
+
+    _say("config", op, case)
+    impl = importlib.import_module(f"tilebench_amd.benchmarks.operators.{op}.impl_hip")
+    names = probe.probe_case(impl, op, case)["names"]
+    cfg = impl.get_last_config()
+    moe = op == "fused_moe_w4a16"
+    products = [n for n in names if re.search(r"w4a16|fp8|moe_gate_up|moe_down|nt_gemm", n)]
+    kernels = cfg["kernels"][2:4] if moe else [cfg["kernel"].split("<")[0]]
+    assert [n.split("<")[0].split("::")[-1] for n in products] == kernels, (names, cfg)
+    for i, name in enumerate(products):
+        if "<" not in name:  # a 256-row kernel
+            assert (cfg["BM"], cfg["BN"]) == (256, 256)
+            continue
+        args = [int({"true": 1, "false": 0}.get(x, x)) for x in re.findall(r"\b(\d+|true|false)\b", name)]
+        kernel = kernels[i]
+        if kernel == "w4a16_decode":
+            assert cfg["cols_per_block"] == 128 * (1 + args[0])
+        elif kernel in ("w4a16_dense", "w4a16_experts"):
+            bn = (cfg["BN_down"] if i else 2 * cfg["BN_gate_up"]) if moe else cfg["BN"]
+            assert (cfg["BM_down"] if moe and i else cfg["BM"], bn) == (32 * args[0], 64 * args[1])
+        elif kernel == "fp8_tile":
+            assert (cfg["BM"], cfg["BN"], cfg["k_groups"]) == (64 * args[0], 64 * args[1], args[4])
+        elif kernel == "fp8_block_gemm":
+            assert (cfg["BM"], cfg["BN"], cfg["waves"]) == (256, args[0], args[1])
+        elif kernel == "nt_gemm":
+            assert cfg["tile"] == f"{args[2]}x{args[3]}"
+        else:
+            assert kernel == "fp8_skinny" and (cfg["BM"], cfg["BN"], cfg["waves"]) == (32, 32, args[0])

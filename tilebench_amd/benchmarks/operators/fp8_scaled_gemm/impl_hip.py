@@ -10,11 +10,11 @@ from tilebench_amd import runtime as rt
 
 rt.load_library()
 
-_last_config = None
+_last_call = None  # (M, N, K)
 
 
 def run(Aq: torch.Tensor, Wq: torch.Tensor, sa: torch.Tensor, sw: torch.Tensor, **kwargs):
-    global _last_config
+    global _last_call
     rt.require_device(Aq, Wq, sa, sw)
     if Aq.dtype != torch.float8_e4m3fn or Wq.dtype != torch.float8_e4m3fn:
         raise TypeError("fp8_scaled_gemm expects float8_e4m3fn operands")
@@ -29,9 +29,9 @@ def run(Aq: torch.Tensor, Wq: torch.Tensor, sa: torch.Tensor, sw: torch.Tensor, 
     Y = torch.empty((M, N), dtype=torch.bfloat16, device=Aq.device)
     rt.call("tb_fp8_scaled_gemm", Aq.data_ptr(), WqT.data_ptr(), sa.data_ptr(), sw.data_ptr(), Y.data_ptr(), M, N, K,
             rt.stream_handle(Aq.device))
-    _last_config = {"kernel": "fp8_gemm_kernel", "BM": "by size", "BN": "by size", "BK": 128}
+    _last_call = M, N, K
     return Y
 
 
 def get_last_config():
-    return _last_config
+    return _last_call and {**rt.gemm_tile(rt.OP_FP8_SCALED, *_last_call), "BK": 128}

@@ -9,7 +9,7 @@ from tilebench_amd import runtime as rt
 
 rt.load_library()
 
-_last_config = None
+_last_call = None  # (pairs, experts, H, I, workspace bytes)
 
 
 def workspace_size(tokens: int, topk: int, experts: int, H: int, I: int) -> int:
@@ -19,7 +19,7 @@ def workspace_size(tokens: int, topk: int, experts: int, H: int, I: int) -> int:
 
 
 def run(X, logits, W13, S13, Z13, W2, S2, Z2, topk: int, group13: int, group2: int, **kwargs):
-    global _last_config
+    global _last_call
     rt.require_device(X, logits, W13, S13, Z13, W2, S2, Z2)
     if X.dtype != torch.float16 or logits.dtype != torch.float32:
         raise TypeError("fused_moe_w4a16 expects fp16 X and fp32 router logits")
@@ -42,10 +42,18 @@ def run(X, logits, W13, S13, Z13, W2, S2, Z2, topk: int, group13: int, group2: i
     rt.call("tb_fused_moe_w4a16", X.data_ptr(), logits.data_ptr(), W13.data_ptr(), S13.data_ptr(), Z13.data_ptr(),
             W2.data_ptr(), S2.data_ptr(), Z2.data_ptr(), out.data_ptr(), T, E, topk, H, I, group13, group2,
             rt.ptr(ws), need, rt.stream_handle(X.device))
-    _last_config = {"kernels": ["gating", "moe_align", "moe_gate_up", "moe_down", "moe_combine"],
-                    "BM": "by size", "BN_gate_up": "by size", "BN_down": "by size", "workspace_bytes": need}
+    _last_call = T * topk, E, H, I, need
     return out
 
 
 def get_last_config():
-    return _last_config
+    """BM and BN of both products (BN_gate_up in activation columns: gate and up
+    columns of a tile are one activation column each)."""
+    if _last_call is None:
+        return None
+    pairs, E, H, I, need = _last_call
+    up = rt.gemm_tile(rt.OP_MOE_GATE_UP, pairs, 2 * I, H, E)
+    down = rt.gemm_tile(rt.OP_MOE_DOWN, pairs, H, I, E)
+    return {"kernels": ["gating", "moe_align", up["kernel"], down["kernel"], "moe_combine"],
+            "BM": up["BM"], "BM_down": down["BM"], "BN_gate_up": up["BN"] // 2, "BN_down": down["BN"],
+            "workspace_bytes": need}

@@ -15,10 +15,12 @@ from tilebench_amd import runtime as rt
 
 rt.load_library()
 
+_last_call = None  # (operator of rt.gemm_tile, M, N, K)
 _DT = {torch.float32: 0, torch.float16: 1, torch.float8_e4m3fn: 2}
 
 
 def run(a: torch.Tensor, b: torch.Tensor, **kwargs):
+    global _last_call
     rt.require_device(a, b)
     if a.dtype not in _DT or b.dtype != a.dtype:
         raise TypeError(f"matmul_fp32_fp16_fp8: unsupported dtypes {a.dtype} / {b.dtype}")
@@ -32,8 +34,12 @@ def run(a: torch.Tensor, b: torch.Tensor, **kwargs):
     need = rt.matmul_workspace_size(dt, M, N, K)
     ws = torch.empty(need, dtype=torch.uint8, device=a.device)
     rt.call("tb_matmul", dt, a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), need, stream)
+    _last_call = rt.OP_MATMUL_F32 + dt, M, N, K
     return out
 
 
 def get_last_config():
-    return {"kernel": "nt_gemm", "tile": "by size"}
+    if _last_call is None:
+        return {"kernel": "nt_gemm"}
+    t = rt.gemm_tile(*_last_call)
+    return {"kernel": t["kernel"], "tile": f"{t['BM']}x{t['BN']}"}

@@ -21,23 +21,16 @@ def run(a: torch.Tensor, b: torch.Tensor, **kwargs):
     ws = torch.empty(need, dtype=torch.uint8, device=a.device)
     rt.call("tb_matmul_int8", a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, ws.data_ptr(), need,
             rt.stream_handle(a.device))
-    global _last_config
-    _last_config = _config(M, N, K)
+    global _last_call
+    _last_call = M, N, K
     return out
 
 
-def _config(M, N, K):
-    """The kernel choice of tb_matmul_int8 (nt_gemm.hip: int8_splits; the tile of
-    an unsplit product is plan::pick_nt_tile's)."""
-    tiles256 = -(-M // 256) * -(-N // 256)
-    splits = 1 if tiles256 >= 256 else min(8, 256 // tiles256, K // 128 // 8)
-    if splits >= 2:
-        return {"kernel": "nt_gemm<i8>", "tile": "256x256", "k_splits": splits}
-    return {"kernel": "nt_gemm<i8>", "tile": "by size", "k_splits": 1}
-
-
-_last_config = None
+_last_call = None  # (M, N, K)
 
 
 def get_last_config():
-    return _last_config
+    if _last_call is None:
+        return None
+    t = rt.gemm_tile(rt.OP_MATMUL_INT8, *_last_call)
+    return {"kernel": f"{t['kernel']}<i8>", "tile": f"{t['BM']}x{t['BN']}", "k_splits": t["k_splits"]}

@@ -5,12 +5,12 @@ from tilebench_amd import runtime as rt
 
 rt.load_library()
 
-_last_config = None
+_last_call = None  # (R, N, K, E)
 
 
 def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, offsets: torch.Tensor,
         group: int, **kwargs):
-    global _last_config
+    global _last_call
     rt.require_device(A, packed, scales, zeros, offsets)
     if A.dtype != torch.float16 or packed.dtype != torch.uint8 or zeros.dtype != torch.uint8 \
             or scales.dtype != torch.float16:
@@ -27,10 +27,14 @@ def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torc
     Y = torch.empty((R, N), dtype=torch.float16, device=A.device)
     rt.call("tb_moe_w4a16_grouped_gemm", A.data_ptr(), packed.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
             offsets.data_ptr(), Y.data_ptr(), R, E, N, K, group, rt.stream_handle(A.device))
-    _last_config = {"kernel": "w4a16_grouped", "BM": "by size", "BN": "by size", "BK": 64,
-                    "last_tiles": "256 x 128 for <= 128 columns"}
+    _last_call = R, N, K, E
     return Y
 
 
 def get_last_config():
-    return _last_config
+    if _last_call is None:
+        return None
+    cfg = {**rt.gemm_tile(rt.OP_W4A16_GROUPED, *_last_call), "BK": 64}
+    if cfg["kernel"] == "w4a16_grouped":
+        cfg["last_tiles"] = "256 x 128 for <= 128 columns"
+    return cfg

@@ -23,7 +23,7 @@ from tilebench_amd.formats import SLAB_COLS, SLAB_UNIT
 
 rt.load_library()
 
-_last_config = None
+_last_call = None  # (layout, M, N, K, workspace bytes)
 
 
 def slab_shape_ok(M: int, N: int, K: int, group: int) -> bool:
@@ -48,7 +48,7 @@ def _weight_shape(packed: torch.Tensor, K: int):
 
 def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, group: int, **kwargs):
     """Y = A @ dequant(packed) in fp16 (fp32 accumulation)."""
-    global _last_config
+    global _last_call
     rt.require_device(A, packed, scales, zeros)
     if A.dtype != torch.float16 or packed.dtype != torch.uint8 or zeros.dtype != torch.uint8 \
             or scales.dtype != torch.float16:
@@ -66,7 +66,7 @@ def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torc
                              f"K in {{1024, 2048, 4096}}, K % 16G == 0); got M={M} K={K} N={N} G={group}")
         rt.call("tb_w4a16_gemm_slabs", A.data_ptr(), packed.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
                 Y.data_ptr(), M, N, K, group, stream)
-        _last_config = {"kernel": "w4a16_slab_decode", "layout": "slabs", "cols_per_block": 64, "waves": 16}
+        _last_call = layout, M, N, K, 0
         return Y
     need = ctypes.c_int64(0)
     if M <= 16:  # only the split-K decode has a workspace
@@ -74,11 +74,18 @@ def run(A: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, zeros: torc
     ws = rt.workspace(need.value, A.device, stream)
     rt.call("tb_w4a16_gemm", A.data_ptr(), packed.data_ptr(), scales.data_ptr(), zeros.data_ptr(), Y.data_ptr(),
             M, N, K, group, rt.ptr(ws), need.value, stream)
-    _last_config = ({"kernel": "w4a16_decode", "layout": "rows", "cols_per_block": "by size",
-                     "workspace_bytes": need.value}
-                    if M <= 16 else {"kernel": "w4a16_prefill", "layout": "rows", "BM": "by size", "BN": "by size", "BK": 64})
+    _last_call = layout, M, N, K, need.value
     return Y
 
 
 def get_last_config():
-    return _last_config
+    if _last_call is None:
+        return None
+    layout, M, N, K, need = _last_call
+    if layout == "slabs":
+        return {"kernel": "w4a16_slab_decode", "layout": "slabs", "cols_per_block": 64, "waves": 16}
+    t = rt.gemm_tile(rt.OP_W4A16, M, N, K)
+    if M <= 16:
+        return {"kernel": t["kernel"], "layout": "rows", "cols_per_block": t["BN"], "k_splits": t["k_splits"],
+                "workspace_bytes": need}
+    return {**t, "layout": "rows", "BK": 64}

@@ -32,6 +32,7 @@
 // 16-byte LDS read; the tile's two columns of weight scales (K/128 values
 // each) are loaded once at the start.
 #include "fp8_small.h"
+#include "gemm_tile.h"
 #include "tb_common.h"
 #include "fp8_codec.h"
 
@@ -439,6 +440,14 @@ extern "C" tb_status tb_fp8_act_quant_blocks(const uint16_t* A, uint8_t* Aq, flo
                      0, stream, reinterpret_cast<const tb::u32x4*>(A), reinterpret_cast<tb::u32x2*>(Aq), sa,
                      (uint32_t)M, (uint32_t)(K / 128));
   return tb::launch_status("tb_fp8_act_quant_blocks");
+}
+
+void tb::describe_fp8_block(int64_t M, int64_t N, int64_t K, tb_tile* out) {
+  const auto tile = plan::pick_fp8_tile(M, N, K, true);
+  if (tile != plan::FP8_256)
+    fp8s::describe_small(tile, true, M, N, out);
+  else
+    *out = tb_tile{"fp8_block_gemm", fp8blk::BM, kLaunchBN, kLaunchWaves, 1, 1};
 }
 
 extern "C" tb_status tb_fp8_block_gemm(const uint8_t* Aq, const uint8_t* WqT, const float* sa, const float* sw,

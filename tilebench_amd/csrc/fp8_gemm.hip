@@ -29,6 +29,7 @@
 // in LDS with 8-byte writes and stores 16-byte row chunks.  Tiles are numbered
 // XCD-aware as in the W4A16 kernel.
 #include "fp8_small.h"
+#include "gemm_tile.h"
 #include "tb_common.h"
 
 #include <type_traits>
@@ -307,6 +308,14 @@ __global__ void __launch_bounds__(THREADS, 1)
 
 }  // namespace fp8gemm
 }  // namespace tb
+
+void tb::describe_fp8_scaled(int64_t M, int64_t N, int64_t K, tb_tile* out) {
+  const auto tile = plan::pick_fp8_tile(M, N, K, false);
+  if (tile != plan::FP8_256)
+    fp8s::describe_small(tile, false, M, N, out);
+  else
+    *out = tb_tile{"fp8_gemm_kernel", fp8gemm::BM, fp8gemm::BN, fp8gemm::THREADS / 64, 1, 1};
+}
 
 extern "C" tb_status tb_fp8_scaled_gemm(const uint8_t* Aq, const uint8_t* WqT, const float* sa, const float* sw,
                                         uint16_t* Y, int64_t M, int64_t N, int64_t K, hipStream_t stream) {

@@ -20,6 +20,9 @@ struct Fp8Args {
   int M, N, K;
 };
 
+// `tile` for tb_gemm_tile.
+void describe_small(plan::Fp8Tile tile, bool block_scaled, int64_t M, int64_t N, tb_tile* out);
+
 tb_status launch_small(const char* fn, plan::Fp8Tile tile, bool block_scaled, const Fp8Args& a, hipStream_t stream);
 
 }  // namespace fp8s

@@ -159,8 +159,9 @@ __global__ void __launch_bounds__(64 * KS, KS / 4 > 0 ? KS / 4 : 1)
 constexpr int MAXKB = 512;
 constexpr uint32_t RSRC_DW3 = 0x00020000u;
 
-template <int FI, int FJ, int ST, bool BLK, int KG>
+template <int FI_, int FJ_, int ST_, bool BLK, int KG_ = 1>
 struct Tile {
+  static constexpr int FI = FI_, FJ = FJ_, ST = ST_, KG = KG_;
   static constexpr int TM = 64 * FI, TN = 64 * FJ;
   static constexpr int A_ST = TM * STEP, STAGE = A_ST + TN * STEP;  // A rows, then W rows
   static constexpr int SA_OFF = ST * STAGE;                         // BLK: the stages' activation scales
@@ -421,29 +422,30 @@ __global__ void __launch_bounds__(256 * KG, 1)
   }
 }
 
+constexpr int SKINNY_KS = 4, SKINNY_D = 2;  // 8 wavefronts or deeper prefetch measured 0 - 5 % slower
+
 template <bool BLK>
 tb_status launch_skinny(const char* fn, const Fp8Args& a, hipStream_t stream) {
-  constexpr int KS = 4, D = 2;  // 8 wavefronts or deeper prefetch measured 0 - 5 % slower
   const int64_t tiles_m = (a.M + 31) / 32, tiles_n = (a.N + TN - 1) / TN;
   TB_CHECK_ARG(tiles_m * tiles_n < (1ll << 31), "%s: problem too large", fn);
-  hipLaunchKernelGGL((fp8_skinny<KS, D, BLK>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * KS), 0, stream, a.Aq,
-                     a.WqT, a.sa, a.sw, a.Y, a.M, a.N, a.K, (int)tiles_m);
+  hipLaunchKernelGGL((fp8_skinny<SKINNY_KS, SKINNY_D, BLK>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * SKINNY_KS), 0,
+                     stream, a.Aq, a.WqT, a.sa, a.sw, a.Y, a.M, a.N, a.K, (int)tiles_m);
   return tb::launch_status(fn);
 }
 
-template <int FI, int FJ, int ST, bool BLK, int KG = 1>
+template <class C, bool BLK>
 tb_status launch_tile(const char* fn, const Fp8Args& a, hipStream_t stream) {
-  typedef Tile<FI, FJ, ST, BLK, KG> C;
-  auto kern = &fp8_tile<FI, FJ, ST, BLK, KG>;
+  auto kern = &fp8_tile<C::FI, C::FJ, C::ST, BLK, C::KG>;
   constexpr size_t lds = C::LDS_BYTES;
   if (tb_status st = tb::reserve_lds(reinterpret_cast<const void*>(kern), lds, fn)) return st;
   const int64_t tiles_m = (a.M + C::TM - 1) / C::TM, tiles_n = (a.N + C::TN - 1) / C::TN;
   TB_CHECK_ARG(tiles_m * tiles_n < (1ll << 31), "%s: problem too large", fn);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256 * KG), lds, stream, a.Aq, a.WqT, a.sa, a.sw, a.Y,
-                     a.M, a.N, a.K, (int)tiles_m);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256 * C::KG), lds, stream, a.Aq, a.WqT, a.sa, a.sw,
+                     a.Y, a.M, a.N, a.K, (int)tiles_m);
   return tb::launch_status(fn);
 }
 
+// f(shape) of an LDS tile: launch and describe take the same one.
 // Ring stages: as deep as pays while one block runs per CU (64 x 64: four, 15.4
 // against 18.9 us with three at 64 x 8192 x 8192; 64 x 128: four, 14.0 against 15.0
 // at 512 x 4096 x 4096); two or three where several tiles share a CU, so that two
@@ -451,26 +453,44 @@ tb_status launch_tile(const char* fn, const Fp8Args& a, hipStream_t stream) {
 // block scales, one block per CU and one wavefront per SIMD, the scale FMAs wait for
 // the MFMAs; two K groups fill each other's waits (200 x 2112 x 7168 17.3 -> 13.8 us,
 // 128 x 8192 x 8192 20.6 -> 16.2, 300 x 5000 x 4096 14.4 -> 13.6; row scales: no gain).
+template <bool BLK, class F>
+tb_status with_tile(plan::Fp8Tile tile, int64_t M, int64_t N, const F& f) {
+  auto tiles = [&](int64_t tm, int64_t tn) { return (M + tm - 1) / tm * ((N + tn - 1) / tn); };
+  switch (tile) {
+    case plan::FP8_64x64:
+      if (BLK && tiles(64, 64) <= 256) return f(Tile<1, 1, 3, BLK, BLK ? 2 : 1>{});
+      return f(Tile<1, 1, BLK ? 3 : 4, BLK>{});
+    case plan::FP8_64x128:
+      if (tiles(64, 128) <= 256) return f(Tile<1, 2, BLK ? 3 : 4, BLK, BLK ? 2 : 1>{});
+      return f(Tile<1, 2, 3, BLK>{});
+    default:
+      if (tiles(128, 128) <= 256) return f(Tile<2, 2, 3, BLK>{});
+      return f(Tile<2, 2, 2, BLK>{});
+  }
+}
+
 template <bool BLK>
 tb_status launch(const char* fn, plan::Fp8Tile tile, const Fp8Args& a, hipStream_t stream) {
-  auto tiles = [&](int64_t tm, int64_t tn) { return (a.M + tm - 1) / tm * ((a.N + tn - 1) / tn); };
-  switch (tile) {
-    case plan::FP8_32x32:
-      return launch_skinny<BLK>(fn, a, stream);
-    case plan::FP8_64x64:
-      if (BLK && tiles(64, 64) <= 256) return launch_tile<1, 1, 3, BLK, BLK ? 2 : 1>(fn, a, stream);
-      return launch_tile<1, 1, BLK ? 3 : 4, BLK>(fn, a, stream);
-    case plan::FP8_64x128:
-      if (tiles(64, 128) <= 256) return launch_tile<1, 2, BLK ? 3 : 4, BLK, BLK ? 2 : 1>(fn, a, stream);
-      return launch_tile<1, 2, 3, BLK>(fn, a, stream);
-    default:
-      if (tiles(128, 128) <= 256) return launch_tile<2, 2, 3, BLK>(fn, a, stream);
-      return launch_tile<2, 2, 2, BLK>(fn, a, stream);
-  }
+  if (tile == plan::FP8_32x32) return launch_skinny<BLK>(fn, a, stream);
+  return with_tile<BLK>(tile, a.M, a.N, [&](auto shape) { return launch_tile<decltype(shape), BLK>(fn, a, stream); });
 }
 
 tb_status launch_small(const char* fn, plan::Fp8Tile tile, bool block_scaled, const Fp8Args& a, hipStream_t stream) {
   return block_scaled ? launch<true>(fn, tile, a, stream) : launch<false>(fn, tile, a, stream);
+}
+
+void describe_small(plan::Fp8Tile tile, bool block_scaled, int64_t M, int64_t N, tb_tile* out) {
+  auto f = [&](auto shape) {
+    typedef decltype(shape) C;
+    *out = tb_tile{"fp8_tile", C::TM, C::TN, 4 * C::KG, C::KG, 1};
+    return TB_OK;
+  };
+  if (tile == plan::FP8_32x32)
+    *out = tb_tile{"fp8_skinny", 32, TN, SKINNY_KS, SKINNY_KS, 1};
+  else if (block_scaled)
+    with_tile<true>(tile, M, N, f);
+  else
+    with_tile<false>(tile, M, N, f);
 }
 
 }  // namespace fp8s

@@ -34,10 +34,12 @@
 // K' = 3K of A' = [A_hi | A_hi | A_lo] and B'^T = [B_hi^T | B_lo^T | B_hi^T],
 // accurate to about 2^-16 per product: finer than the TF32 the reference
 // allows for its fp32 matmul (10 mantissa bits) and run at the bf16 rate.
+#include "gemm_tile.h"
 #include "small_plan.h"
 #include "tb_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace tb {
 namespace ntg {
@@ -760,30 +762,55 @@ tb_status launch_small(const uint8_t* A, const uint8_t* BT, void* Y, int64_t M, 
   return launch_status(what);
 }
 
-// The product on the tile plan::pick_nt_tile picks.  Ring stages: four of 64 x 64
+// f(tile rows / 64, tile columns / 64, stages) of a small pick: launch and describe
+// take the same one.  Ring stages: four of 64 x 64
 // (16 x 4096 x 4096 fp16 14.7 against 16.5 us with three), three otherwise, two
 // where several 128 x 128 tiles share a CU so that two blocks fit (1690 x 3432 x
 // 2176 fp16 34 against 40 us).
+template <class F>
+tb_status with_small(plan::NtTile tile, int64_t M, int64_t N, const F& f) {
+  typedef std::integral_constant<int, 1> I1;
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 3> I3;
+  switch (tile) {
+    case plan::NT_64x64:
+      return f(I1{}, I1{}, std::integral_constant<int, 4>{});
+    case plan::NT_64x128:
+      return f(I1{}, I2{}, I3{});
+    default:
+      if (((M + 127) / 128) * ((N + 127) / 128) <= 256) return f(I2{}, I2{}, I3{});
+      return f(I2{}, I2{}, I2{});
+  }
+}
+
+// The product on the tile plan::pick_nt_tile picks.
 template <int KIND, int OUT>
 tb_status launch_any(const uint8_t* A, const uint8_t* BT, void* Y, int64_t M, int64_t N, int64_t Kb,
                      hipStream_t stream, const char* what) {
   // e4m3 rows are stored in 8-byte granules by the small tiles, in 4-byte ones by nt_gemm
   const plan::NtTile tile = OUT == OUT_E4M3 && !aligned(Y, 8) ? plan::NT_256 : plan::pick_nt_tile(M, N, Kb);
-  switch (tile) {
-    case plan::NT_64x64:
-      return launch_small<KIND, OUT, 1, 1, 4>(A, BT, Y, M, N, Kb, stream, what);
-    case plan::NT_64x128:
-      return launch_small<KIND, OUT, 1, 2, 3>(A, BT, Y, M, N, Kb, stream, what);
-    case plan::NT_128x128:
-      if (((M + 127) / 128) * ((N + 127) / 128) <= 256)
-        return launch_small<KIND, OUT, 2, 2, 3>(A, BT, Y, M, N, Kb, stream, what);
-      return launch_small<KIND, OUT, 2, 2, 2>(A, BT, Y, M, N, Kb, stream, what);
-    default:
-      return launch_nt<KIND, OUT, 256, 256, 128, 64>(A, BT, Y, nullptr, nullptr, M, N, Kb, stream, what);
-  }
+  if (tile == plan::NT_256)
+    return launch_nt<KIND, OUT, 256, 256, 128, 64>(A, BT, Y, nullptr, nullptr, M, N, Kb, stream, what);
+  return with_small(tile, M, N, [&](auto fi, auto fj, auto st) {
+    return launch_small<KIND, OUT, decltype(fi)::value, decltype(fj)::value, decltype(st)::value>(A, BT, Y, M, N, Kb,
+                                                                                                 stream, what);
+  });
 }
 
 }  // namespace ntg
+
+void describe_matmul(int op, int64_t M, int64_t N, int64_t K, tb_tile* out) {
+  // bytes of K per operand row (fp32: three bf16 terms)
+  const int64_t kb = op == TB_OP_MATMUL_F32 ? 6 * K : op == TB_OP_MATMUL_F16 ? 2 * K : K;
+  const int splits = op == TB_OP_MATMUL_INT8 ? ntg::int8_splits(M, N, K) : 1;
+  const plan::NtTile tile = splits > 1 ? plan::NT_256 : plan::pick_nt_tile(M, N, kb);
+  *out = tb_tile{"nt_gemm", 256, 256, 8, 1, splits};
+  if (tile != plan::NT_256)
+    ntg::with_small(tile, M, N, [&](auto fi, auto fj, auto) {
+      *out = tb_tile{"nt_gemm", 64 * fi, 64 * fj, 4, 1, 1};
+      return TB_OK;
+    });
+}
 }  // namespace tb
 
 using namespace tb::ntg;

@@ -1,5 +1,6 @@
-// Library-level entry points: version, error reporting, the cache-flush fill
-// kernel and the HBM streaming-copy probe.
+// Library-level entry points: version, error reporting, the tile of a GEMM call,
+// the cache-flush fill kernel and the HBM streaming-copy probe.
+#include "gemm_tile.h"
 #include "tb_common.h"
 
 #include <string.h>
@@ -259,6 +260,24 @@ tb_status tb_probe_copy(const void* src, void* dst, int64_t bytes, hipStream_t s
   hipLaunchKernelGGL(tb::copy_kernel, dim3(tb::grid_for(n16)), dim3(256), 0, stream,
                      reinterpret_cast<const tb::u32x4*>(src), reinterpret_cast<tb::u32x4*>(dst), n16);
   return tb::launch_status("tb_probe_copy");
+}
+
+tb_status tb_gemm_tile(int op, int64_t M, int64_t N, int64_t K, int64_t experts, tb_tile* tile) {
+  TB_CHECK_ARG(tile != nullptr, "tb_gemm_tile: null output");
+  TB_CHECK_ARG(op >= TB_OP_W4A16 && op <= TB_OP_MATMUL_INT8, "tb_gemm_tile: unknown operator %d", op);
+  const bool expert_op = op >= TB_OP_W4A16_GROUPED && op <= TB_OP_MOE_DOWN;
+  TB_CHECK_ARG(M > 0 && N > 0 && K > 0 && (experts > 0 || !expert_op), "tb_gemm_tile: sizes must be positive");
+  if (op == TB_OP_W4A16)
+    tb::describe_w4a16(M, N, K, tile);
+  else if (expert_op)
+    tb::describe_experts(op, M, N, experts, tile);
+  else if (op == TB_OP_FP8_SCALED)
+    tb::describe_fp8_scaled(M, N, K, tile);
+  else if (op == TB_OP_FP8_BLOCK)
+    tb::describe_fp8_block(M, N, K, tile);
+  else
+    tb::describe_matmul(op, M, N, K, tile);
+  return TB_OK;
 }
 
 }  // extern "C"

@@ -52,6 +52,7 @@
 // contiguous run of tiles, and runs are ordered in groups of 4 tile rows, so
 // the blocks resident on one XCD share A rows and W columns in its L2.
 #include "tb_common.h"
+#include "gemm_tile.h"
 #include "prefill_plan.h"
 #include "w4a16_small.h"
 #include "w4a16_tile.h"
@@ -1465,6 +1466,31 @@ static tb_status scratch_of_current_device(const char* fn, hipStream_t stream, v
 }
 
 }  // namespace w4a16
+
+void describe_w4a16(int64_t M, int64_t N, int64_t K, tb_tile* out) {
+  using namespace w4a16;
+  if (M <= 16) {
+    const plan::DecodePlan p = decode_plan(N, K);
+    *out = tb_tile{"w4a16_decode", 16, p.cols, DEC_WAVES, DEC_WAVES, p.splits};
+    return;
+  }
+  const auto tile = plan::pick_dense_tile(M, N);
+  if (tile != plan::DENSE_256)
+    describe_dense_small(tile, M, out);
+  else
+    *out = tb_tile{"w4a16_prefill", BM, BN, 4, 1, 1};
+}
+
+void describe_experts(int op, int64_t rows, int64_t N, int64_t experts, tb_tile* out) {
+  using namespace w4a16;
+  const auto tile = plan::pick_expert_tile(rows, experts, N);
+  if (tile != plan::TILE_256)
+    describe_experts_small(tile, out);
+  else if (op == TB_OP_MOE_DOWN)
+    *out = tb_tile{"moe_down", BM, BN, p8::THREADS / 64, 1, 1};
+  else
+    *out = tb_tile{op == TB_OP_MOE_GATE_UP ? "moe_gate_up" : "w4a16_grouped", BM, BN, 4, 1, 1};
+}
 }  // namespace tb
 
 extern "C" tb_status tb_w4a16_gemm(const uint16_t* A, const uint8_t* W, const uint16_t* scales, const uint8_t* zeros,

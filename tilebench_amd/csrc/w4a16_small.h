@@ -35,6 +35,10 @@ struct ExpertArgs {
   int experts, N, K, group;
 };
 
+// `tile` for tb_gemm_tile.
+void describe_dense_small(plan::DenseTile tile, int64_t M, tb_tile* out);
+void describe_experts_small(plan::ExpertTile tile, tb_tile* out);
+
 tb_status launch_dense_small(const char* fn, plan::DenseTile tile, const DenseArgs& a, hipStream_t stream);
 
 // Arguments checked by the caller (the limits of the 256-row kernels).

@@ -551,25 +551,21 @@ tb_status launch_shape(const char* fn, const ExpertArgs& a, hipStream_t stream) 
   return tb::launch_status(fn);
 }
 
-template <int MODE>
-tb_status launch_mode(const char* fn, plan::ExpertTile tile, const ExpertArgs& a, hipStream_t stream) {
-  // 16-byte W DMAs need every K row of every expert, and in gate/up the up half
-  // of a row, to start on 16 bytes
-  const bool wide = tb::aligned(a.W, 16) && a.N % (MODE == T_GATE_UP ? 64 : 32) == 0;
+// f(shape) of a pick: launch and describe take the same one.
+template <class F>
+tb_status with_expert_shape(plan::ExpertTile tile, const F& f) {
   switch (tile) {
     case plan::TILE_32x128:
-      return wide ? launch_shape<S32x128, true, MODE>(fn, a, stream) : launch_shape<S32x128, false, MODE>(fn, a, stream);
+      return f(S32x128{});
     case plan::TILE_32x256:
-      return wide ? launch_shape<S32x256, true, MODE>(fn, a, stream) : launch_shape<S32x256, false, MODE>(fn, a, stream);
+      return f(S32x256{});
     default:
-      return wide ? launch_shape<S64x256, true, MODE>(fn, a, stream) : launch_shape<S64x256, false, MODE>(fn, a, stream);
+      return f(S64x256{});
   }
 }
-}  // namespace sm
 
-tb_status launch_dense_small(const char* fn, plan::DenseTile tile, const DenseArgs& a, hipStream_t stream) {
-  using namespace sm;
-  const bool wide = tb::aligned(a.W, 16) && a.N % 32 == 0;
+template <class F>
+tb_status with_dense_shape(plan::DenseTile tile, int64_t M, const F& f) {
   switch (tile) {
     case plan::DENSE_64x64_K4:
       // Up to 32 rows half of a 64-row tile's MFMAs, A DMAs and A reads are padding
@@ -577,16 +573,48 @@ tb_status launch_dense_small(const char* fn, plan::DenseTile tile, const DenseAr
       // counts gained nothing).  The same K groups in the same order: the bits are those of
       // the 64-row tile.  Kernel, us, 64 -> 32 rows: 32 x 11008 (K 4096) 13.9 -> 12.5, 24 x
       // 4096 (K 11008) 33.2 -> 29.0, 20 x 12288 (K 1024) 7.3 -> 6.3.
-      if (a.M <= 32)
-        return wide ? launch_dense_shape<S32x64k4, true>(fn, a, stream) : launch_dense_shape<S32x64k4, false>(fn, a, stream);
-      return wide ? launch_dense_shape<S64x64k4, true>(fn, a, stream) : launch_dense_shape<S64x64k4, false>(fn, a, stream);
+      return M <= 32 ? f(S32x64k4{}) : f(S64x64k4{});
     case plan::DENSE_64x128:
-      return wide ? launch_dense_shape<S64x128, true>(fn, a, stream) : launch_dense_shape<S64x128, false>(fn, a, stream);
+      return f(S64x128{});
     case plan::DENSE_64x256:
-      return wide ? launch_dense_shape<S64x256, true>(fn, a, stream) : launch_dense_shape<S64x256, false>(fn, a, stream);
+      return f(S64x256{});
     default:
-      return wide ? launch_dense_shape<S128x256, true>(fn, a, stream) : launch_dense_shape<S128x256, false>(fn, a, stream);
+      return f(S128x256{});
   }
+}
+
+template <class C>
+tb_status describe(const char* kernel, tb_tile* out) {
+  *out = tb_tile{kernel, C::TM, C::TN, C::THREADS / 64, C::KS, 1};
+  return TB_OK;
+}
+
+template <int MODE>
+tb_status launch_mode(const char* fn, plan::ExpertTile tile, const ExpertArgs& a, hipStream_t stream) {
+  // 16-byte W DMAs need every K row of every expert, and in gate/up the up half
+  // of a row, to start on 16 bytes
+  const bool wide = tb::aligned(a.W, 16) && a.N % (MODE == T_GATE_UP ? 64 : 32) == 0;
+  return with_expert_shape(tile, [&](auto shape) {
+    typedef decltype(shape) C;
+    return wide ? launch_shape<C, true, MODE>(fn, a, stream) : launch_shape<C, false, MODE>(fn, a, stream);
+  });
+}
+}  // namespace sm
+
+void describe_dense_small(plan::DenseTile tile, int64_t M, tb_tile* out) {
+  sm::with_dense_shape(tile, M, [&](auto shape) { return sm::describe<decltype(shape)>("w4a16_dense", out); });
+}
+
+void describe_experts_small(plan::ExpertTile tile, tb_tile* out) {
+  sm::with_expert_shape(tile, [&](auto shape) { return sm::describe<decltype(shape)>("w4a16_experts", out); });
+}
+
+tb_status launch_dense_small(const char* fn, plan::DenseTile tile, const DenseArgs& a, hipStream_t stream) {
+  const bool wide = tb::aligned(a.W, 16) && a.N % 32 == 0;
+  return sm::with_dense_shape(tile, a.M, [&](auto shape) {
+    typedef decltype(shape) C;
+    return wide ? sm::launch_dense_shape<C, true>(fn, a, stream) : sm::launch_dense_shape<C, false>(fn, a, stream);
+  });
 }
 
 tb_status launch_experts_small(const char* fn, TileMode mode, plan::ExpertTile tile, const ExpertArgs& a,

@@ -30,6 +30,17 @@ _c_p = ctypes.c_void_p
 _c_int = ctypes.c_int
 _c_u32 = ctypes.c_uint32
 
+class GemmTile(ctypes.Structure):
+    """tb_tile: the kernel and tile of a GEMM call."""
+
+    _fields_ = [("kernel", ctypes.c_char_p), ("tile_rows", ctypes.c_int32), ("tile_cols", ctypes.c_int32),
+                ("wavefronts", ctypes.c_int32), ("k_groups", ctypes.c_int32), ("k_splits", ctypes.c_int32)]
+
+
+#: tb_gemm_tile's operators
+(OP_W4A16, OP_W4A16_GROUPED, OP_MOE_GATE_UP, OP_MOE_DOWN, OP_FP8_SCALED, OP_FP8_BLOCK, OP_MATMUL_F32, OP_MATMUL_F16,
+ OP_MATMUL_FP8, OP_MATMUL_INT8) = range(10)
+
 #: symbol -> argtypes (every entry point returns an int status).
 SIGNATURES: dict[str, list] = {
     "tb_int4_dequant": [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p],
@@ -57,6 +68,7 @@ SIGNATURES: dict[str, list] = {
     "tb_matmul": [_c_int, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p],
     "tb_matmul_fp8_bt": [_c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p],
     "tb_matmul_workspace_size": [_c_int, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_i64)],
+    "tb_gemm_tile": [_c_int, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.POINTER(GemmTile)],
     "tb_l2_flush": [_c_p, _c_i64, _c_u32, _c_p],
     "tb_probe_copy": [_c_p, _c_p, _c_i64, _c_p],
     "tb_probe_read": [_c_p, _c_i64, _c_u32, _c_p, _c_p],
@@ -172,6 +184,15 @@ def matmul_workspace_size(dtype: int, M: int, N: int, K: int) -> int:
     out = ctypes.c_int64(0)
     call("tb_matmul_workspace_size", dtype, M, N, K, ctypes.byref(out))
     return int(out.value)
+
+
+def gemm_tile(op: int, M: int, N: int, K: int, experts: int = 0) -> dict:
+    """The kernel and tile a GEMM call of these sizes launches (tb_gemm_tile):
+    asked for when a configuration is read, so a call pays nothing for it."""
+    t = GemmTile()
+    call("tb_gemm_tile", op, M, N, K, experts, ctypes.byref(t))
+    return {"kernel": t.kernel.decode(), "BM": t.tile_rows, "BN": t.tile_cols, "waves": t.wavefronts,
+            "k_groups": t.k_groups, "k_splits": t.k_splits}
 
 
 def workspace(nbytes: int, device, stream: int):
