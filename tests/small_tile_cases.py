@@ -17,9 +17,11 @@ EXPERT_TILE_IDS = {"256": 0, "32x128": 1, "32x256": 2, "64x256": 3}
 DENSE_TILES = {
     "64x64": [(17, 64, 8, 64), (33, 320, 392, 64), (64, 704, 1000, 64), (48, 2048, 4096, 128)],
     "64x128": [(65, 64, 264, 64), (129, 448, 1096, 64), (500, 192, 4096, 64)],
-    "64x256": [(691, 192, 11896, 64), (1000, 128, 4096, 64)],
+    "64x256": [(300, 192, 22040, 64), (1000, 128, 4096, 64)],
     "128x256": [(768, 320, 8944, 64), (2047, 64, 4096, 64)],
-    "256": [(1024, 192, 11008, 64)],
+    # half a round and more of 256 x 256 tiles: two rounds and a bit of a smaller tile take 20 - 28 % longer
+    "256": [(1024, 192, 11008, 64), (691, 192, 11896, 64), (729, 64, 12288, 64), (1725, 64, 5480, 64),
+            (2204, 64, 4096, 64), (4086, 64, 2216, 64)],
 }
 DENSE_TILE_IDS = {"256": 0, "64x64": 1, "64x128": 2, "64x256": 3, "128x256": 4}
 

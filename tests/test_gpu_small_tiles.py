@@ -115,14 +115,17 @@ def test_dense_tiles_match_oracle(gpu, tile):
                                    rtol=1e-2)
 
 
-@pytest.mark.parametrize("M", [65, 500, 900])  # 64 x 128, 128 x 256 and 64 x 256 tiles
-def test_dense_rows_do_not_depend_on_the_tile(gpu, M):
+@pytest.mark.parametrize("M,N,tile", [(65, 11008, (64, 128)), (500, 11008, (128, 256)), (300, 22040, (64, 256))])
+def test_dense_rows_do_not_depend_on_the_tile(gpu, M, N, tile):
     """More than 64 rows: the first M rows alone give the bits they have in a
     product of 256 x 256 tiles.  64 rows (K in four groups) are reproducible."""
     from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
 
-    A, p, s, z, G = T.generate_w4a16_gemm_inputs(1024, 448, 11008 if M != 900 else 10752, 64, seed=3, device="cpu")
-    _say("dense rows", M)
+    A, p, s, z, G = T.generate_w4a16_gemm_inputs(1024, 448, N, 64, seed=3, device="cpu")
+    _say("dense rows", M, N)
+    for m, t in ((M, tile), (1024, (256, 256))):
+        picked = rt.gemm_tile(rt.OP_W4A16, m, N, 448)
+        assert (picked["BM"], picked["BN"]) == t
     A, p, s, z = (t.to(gpu) for t in (A, p, s, z))
     big = impl_hip.run(A, p, s, z, G)
     small = impl_hip.run(A[:M].contiguous(), p, s, z, G)

@@ -10,6 +10,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 namespace tb {
@@ -52,31 +53,48 @@ inline ExpertTile pick_expert_tile(int64_t rows, int64_t experts, int64_t N) {
 
 enum DenseTile { DENSE_256 = 0, DENSE_64x64_K4, DENSE_64x128, DENSE_64x256, DENSE_128x256 };
 
-// The tile of a dense product of more than 16 rows, by the same estimate (us per
-// K step, measured at K = 4096 and 11008 on 43 - 1376 tiles).  Up to 64 rows
-// 64-column tiles of four K groups put a product on every CU that has columns
-// for it: 48 rows x 11008 columns 15 us against 25 (64 x 128), 30 (64 x 256)
+// us of a K step of `x` tiles per CU, as it was measured: a line over the first
+// round of tiles, then a stair per round (a round that is nearly empty costs nearly
+// as much as a full one) with a slope for how full the last one is.  `power` is for
+// the 256 x 256 tiles, whose clock falls with the share of the chip that multiplies
+// (`work`: tiles per CU without their padding).
+struct Stairs {
+  double first, slope, second, round, fill, power = 0;
+  double operator()(double x, double work = 0) const {
+    if (x <= 1) return first + slope * x + power * std::max(0.0, work - 0.3);
+    const double rounds = std::ceil(x);
+    return second + round * (rounds - 2) + fill * (x - (rounds - 1));
+  }
+};
+
+// The tile of a dense product of more than 16 rows, by the same estimate.  The
+// constants are least-squares fits over sizes of 17 - 8192 rows, K and N 64 - 32768 (cold
+// weights, each tile forced in turn): within 7 % of nine in ten.  The 256 x 256
+// tiles are priced 2 % below their fit, so that a tie goes to them.  Over 5177 sizes the
+// picks then took 0.2 % more than the best tile, and two over 3 % more than 256 x 256
+// (636 x 28552, K 2368: 102 us against 97).
+// Up to 64 rows 64-column tiles of four K groups put a product on every CU that has
+// columns for it: 48 rows x 11008 columns 15 us against 25 (64 x 128), 30 (64 x 256)
 // and 62 (256 x 256); up to 32 rows the launch halves its rows (12.5 at 32 rows,
-// 13.9 on 64).  128 x 11008 (K = 4096): 64 x 128 25 us, 64 x 256 31, 128
-// x 256 42, 256 x 256 63; 512 x 11008: 61 / 59 / 52 / 71; 1024 x 11008: 116 /
-// 101 / 106 / 95; 500 x 4096 (K = 11008): 65 / 78 / 106 / 160.
+// 13.9 on 64).  500 x 4096 (K = 11008): 64 x 128 65 us, 64 x 256 78, 128 x 256 106,
+// 256 x 256 160.  Half a round of 256 x 256 tiles beats two rounds and a bit of any
+// smaller one: 729 x 12288 (K = 4096) 72 us against 91 (64 x 256), 2391 x 3608 (K =
+// 10560) 193 against 247 (128 x 256).
 inline DenseTile pick_dense_tile(int64_t M, int64_t N) {
   auto tiles = [&](int64_t tm, int64_t tn) { return (double)((M + tm - 1) / tm * ((N + tn - 1) / tn)) / 256.0; };
-  // x: tiles per CU
-  auto c64 = [](double x) { return 0.18 * std::max(1.0, x); };
-  auto c128 = [](double x) { return x <= 1 ? 0.30 + 0.05 * x : std::max(0.5, 0.32 * x); };
-  auto c256 = [](double x) { return x <= 1 ? 0.40 + 0.10 * x : std::max(0.83, 0.55 * x); };
-  auto c128x256 = [](double x) { return x <= 1 ? 0.56 + 0.25 * x : std::max(1.56, x); };  // one tile per CU
-  auto cbig = [](double x) { return x <= 1 ? 0.80 + 0.85 * x : std::max(2.66, 1.74 * x); };
+  constexpr double steps = 64;  // K = 4096: the start and end of a tile weigh little beside its steps
+  constexpr Stairs s64{0.11, 0.20, 0.62, 0.25, 0}, s128{0.30, 0.07, 0.48, 0.33, 0.18},
+      s256{0.41, 0.15, 0.82, 0.56, 0.26}, s128x256{0.56, 0.30, 1.49, 1.02, 0.38},
+      sbig{0.86, 0.26, 2.40, 1.77, 0.83, 0.72};
   DenseTile best = DENSE_256;
-  double c = cbig(tiles(256, 256));
+  double c = 0.98 * (6 + steps * sbig(tiles(256, 256), (double)M * (double)N / 65536.0 / 256.0));
   auto take = [&](DenseTile t, double cost) {
     if (cost < c) best = t, c = cost;
   };
-  take(DENSE_128x256, c128x256(tiles(128, 256)));
-  take(DENSE_64x256, c256(tiles(64, 256)));
-  take(DENSE_64x128, c128(tiles(64, 128)));
-  if (M <= 64) take(DENSE_64x64_K4, c64(tiles(64, 64)));
+  take(DENSE_128x256, 5 + steps * s128x256(tiles(128, 256)));
+  take(DENSE_64x256, 4 + steps * s256(tiles(64, 256)));
+  take(DENSE_64x128, 4 + steps * s128(tiles(64, 128)));
+  if (M <= 64) take(DENSE_64x64_K4, 4 + steps * s64(tiles(64, 64)));
   return best;
 }
 
