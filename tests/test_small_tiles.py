@@ -60,16 +60,21 @@ def test_decode_plans_picked(tmp_path):
     def picks(cases):
         args = [str(x) for cus, K, N in cases for x in (cus, -2 * 10 ** 9 - K, N)]
         out = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-        return [(int(g) // 1000, int(g) % 1000) for g in out]
+        return [(int(g) % 10 ** 9 // 1000, int(g) % 1000, int(g) // 10 ** 9) for g in out]
 
     listed = [(plan, 256, K, N) for plan, cs in DECODE_PLANS.items() for N, K in cs]
-    assert picks([c[1:] for c in listed]) == [c[0] for c in listed]
+    assert [p[:2] for p in picks([c[1:] for c in listed])] == [c[0] for c in listed]
     cases = [(cus, K, N) for cus in (1, 64, 256, 304) for K in (64, 192, 256, 1024, 7168, 32768)
              for N in (8, 128, 1000, 4096, 32768, 32776, 65536)]
-    for (cus, K, N), (cols, splits) in zip(cases, picks(cases)):
+    # pairs of 128-column slabs that do not divide over the 8 XCDs: five splits of 26 pairs
+    # would be 34 blocks on some XCDs of 32 CUs, three of 43 likewise
+    cases += [(256, 9920, 6528), (256, 4096, 10880), (256, 7744, 6448), (256, 2560, 10816), (256, 12672, 3136)]
+    for (cus, K, N), (cols, splits, blocks) in zip(cases, picks(cases)):
         slabs = -(-N // cols)
         assert cols in (128, 256) and 1 <= splits <= 16
         assert splits == 1 or (slabs * splits <= cus and splits * 8 <= K // 32)
+        assert blocks == (2 * 8 * -(-(-(-slabs // 2) * splits) // 8) if cols == 128 else slabs * splits)
+        assert splits == 1 or blocks <= cus  # the launched grid, and with it every XCD's share
 
 
 def test_reported_tiles_are_the_picked_ones():

@@ -177,7 +177,14 @@ struct DecodePlan {
 // 7.8 / 11.4; K 4096, N 11008 11.4 / 12.5; K 4096, N 12288 13.5 / 13.2; K 8192, N
 // 28672 43.1 / 32.6.  Splits at 128
 // columns, K 4096, N 4096: 1 13.1, 2 9.7, 4 7.8, 8 8.5; K 1024, N 12288: 1 6.0, 2 6.7.
-// A split grid never has more blocks than CUs.
+// A split grid never has more blocks than CUs, counted as they are launched: pairs of
+// 128-column slabs go to the 8 XCDs in turn, and a block fills a CU, so a pair too many on
+// one XCD would start its blocks a whole block's time later (9 x 6528, K 9920, five splits
+// of 51 slabs, 34 blocks on an XCD of 32 CUs: 19.6 us; 256-column slabs 16.1, now 14.0).
+inline int64_t decode_grid(int cols, int64_t slabs, int splits) {
+  return cols == 128 ? ((slabs + 1) / 2 * splits + 7) / 8 * 16 : slabs * splits;
+}
+
 inline DecodePlan pick_decode(int64_t N, int64_t K, int cus) {
   const int64_t units = K / DEC_UNIT;
   DecodePlan best{128, (N + 127) / 128, 1};
@@ -185,7 +192,7 @@ inline DecodePlan pick_decode(int64_t N, int64_t K, int cus) {
   for (int cols = 128; cols <= (N <= 128 ? 128 : 256); cols += 128) {  // the wide slab needs 16 columns
     const bool wide = cols == 256;
     const int64_t slabs = (N + cols - 1) / cols;
-    for (int s = 1; s <= DEC_MAX_SPLITS && (s == 1 || (slabs * s <= cus && (int64_t)s * DEC_WAVES <= units)); ++s) {
+    for (int s = 1; s <= DEC_MAX_SPLITS && (s == 1 || (decode_grid(cols, slabs, s) <= cus && (int64_t)s * DEC_WAVES <= units)); ++s) {
       const double rounds = (double)((slabs * s + cus - 1) / cus), share = (double)units / (s * DEC_WAVES);
       double cost = wide ? rounds * std::max(1.0, share) * 1.45
                          : rounds * (double)(int64_t)(share + 0.999999) * 0.75 + 0.055e-6 * (double)N * (double)K;

@@ -1385,16 +1385,16 @@ static tb_status launch_dense(const char* fn, const uint16_t* A, const uint8_t* 
     int* counters = reinterpret_cast<int*>(workspace);
     float* partials =
         p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + DEC_COUNTER_BYTES) : nullptr;
-    auto launch = [&](auto kern, int64_t blocks) {
-      hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(DEC_THREADS), 0, stream,
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)plan::decode_grid(p.cols, p.slabs, p.splits)), dim3(DEC_THREADS), 0, stream,
                          reinterpret_cast<const _Float16*>(A), W, reinterpret_cast<const _Float16*>(scales), zeros,
                          reinterpret_cast<_Float16*>(Y), partials, counters, (int)M, (int)N, (int)K, (int)group,
                          p.splits);
     };
     if (p.cols == 128)
-      launch(w4a16_decode<false>, ((p.slabs + 1) / 2 * p.splits + 7) / 8 * 16);
+      launch(w4a16_decode<false>);
     else
-      launch(w4a16_decode<true>, p.slabs * p.splits);
+      launch(w4a16_decode<true>);
     return tb::launch_status(fn);
   }
   const auto tile = tb::plan::pick_dense_tile(M, N);
