@@ -42,7 +42,8 @@ FP8_TILE_IDS = {"256": 0, "32x32": 1, "64x64": 2, "64x128": 3, "128x128": 4}
 NT_TILES = {
     "64x64": [(1, 8, 128), (65, 1000, 640), (100, 4104, 1152)],
     "64x128": [(513, 2056, 640), (300, 5000, 384)],
-    "128x128": [(1000, 2104, 1152), (1100, 5000, 640)],
+    # the last two: just over one tile per CU on many steps, and half a round of 256 x 256 tiles on few
+    "128x128": [(1000, 2104, 1152), (1100, 5000, 640), (3380, 1192, 3840), (2779, 3616, 256)],
     "256": [(4096, 4104, 1152)],
 }
 NT_TILE_IDS = {"256": 0, "64x64": 1, "64x128": 2, "128x128": 3}

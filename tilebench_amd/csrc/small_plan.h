@@ -138,23 +138,28 @@ inline Fp8Tile pick_fp8_tile(int64_t M, int64_t N, int64_t K, bool block_scaled)
 enum NtTile { NT_256 = 0, NT_64x64, NT_64x128, NT_128x128 };
 
 // The tile of a plain product (Kb: bytes of K per operand row), by the same
-// estimate: a step of 128 bytes takes 0.2 us at 64 x 64, 0.31 at 64 x 128, 0.4 -
-// 0.6 at 128 x 128 and 1.35 - 1.95 at 256 x 256 (fp16; the other types within a
-// fifth).  Measured fp16 products alone, us: 16 x 4096 x 4096 14.7 (64 x 64;
+// estimate: a step of 128 bytes takes 0.2 us at 64 x 64, 0.31 at 64 x 128, 0.36 -
+// 0.54 at 128 x 128 (two of them share a CU and step in 0.75 - 1.1, not in twice that)
+// and 1.35 - 1.95 at 256 x 256, whose start and end take 4 us more than a small tile's
+// (fp16 and fp32; the others within a fifth).  Over 3018 sizes of the four types the picks
+// take 0.3 % more than the best tile; without those two terms fp32 3380 x 1192 x 3968 ran
+// on 64 x 64 tiles (177 us, 128 x 128 156) and int8 2779 x 3616 x 256 on 256 x 256
+// (22.7, 128 x 128 19.6).  Measured fp16 products alone, us: 16 x 4096 x 4096 14.7 (64 x 64;
 // 256 x 256 86), 512 x 4096 x 4096 23.4 (64 x 128; 93), 2048 x 2048 x 4096 39 (128 x
-// 128; 95), 2601 x 1648 x 2432 30 (128 x 128; 58), 3362 x 2504 x 5248 120 (256 x
-// 256; 128 x 128 128), 4096 x 4096 x 4096 129 (256 x 256; 128 x 128 135).
+// 128; 95), 2601 x 1648 x 2432 30 (128 x 128; 58), 2872 x 3104 x 5504 with its
+// transpose 155 (128 x 128; 256 x 256 158), 4096 x 4096 x 4096 129 (256 x 256; 128 x 128 135).
 inline NtTile pick_nt_tile(int64_t M, int64_t N, int64_t Kb) {
   const double s = (double)Kb / 128;
   auto tiles = [&](int64_t tm, int64_t tn) { return (double)((M + tm - 1) / tm * ((N + tn - 1) / tn)) / 256.0; };
   auto up = [](double v) { return (double)(int64_t)(v + 0.999999); };
   const double big = tiles(256, 256), t128 = tiles(128, 128), t64x128 = up(tiles(64, 128)), t64 = up(tiles(64, 64));
-  double c = 3 * std::max(1.0, big) + s * (big <= 1 ? 1.35 + 0.2 * big + std::max(0.0, big - 0.6) : 1.95 * big);
+  double c = 4 + 3 * std::max(1.0, big) + s * (big <= 1 ? 1.35 + 0.2 * big + std::max(0.0, big - 0.6) : 1.95 * big);
   NtTile best = NT_256;
   auto take = [&](NtTile t, double cost) {
     if (cost < c) best = t, c = cost;
   };
-  take(NT_128x128, 3 * std::max(1.0, t128 / 2) + s * (t128 <= 1 ? 0.4 + 0.2 * t128 : t128 <= 2 ? 0.9 : std::max(1.6, 0.53 * t128)));
+  constexpr Stairs s128{0.36, 0.18, 0.75, 0.65, 0.35};
+  take(NT_128x128, 3 * std::max(1.0, up(t128) / 2) + s * s128(t128));
   take(NT_64x128, 3 * std::max(1.0, t64x128 / 2) + s * (0.30 * t64x128 + 0.03));
   take(NT_64x64, 3 * std::max(1.0, t64 / 2) + s * std::max(0.2, 0.19 * t64));
   return best;
