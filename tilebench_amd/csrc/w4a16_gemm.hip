@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, kg = lane >> 4;
   // A lane of 16 columns whose last 8 do not exist (N % 16 == 8) also takes the 8 before
-  // its first, its neighbour's, so that every load is whole; it stages only its own.
+  // its first, its neighbour's, so that every load is whole; only its own are stored.
   const bool col_ok = n0 + c * CPL < N;  // at least 8 columns exist (N % 8 == 0)
   const int extra = WIDE && col_ok && n0 + c * CPL + CPL > N ? 8 : 0;
   const int n = n0 + c * CPL - extra;    // >= 0: N = 8 takes 128-column slabs
@@ -287,17 +287,18 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
     fold(tmp, asum, gp);
   }
 
-  // Accumulator f, element e: row 4 * (lane / 16) + e, column CPL c + f.  A row's
-  // 16-byte chunks are ordered by f / 4, then c, so that the 16 lanes of a write
-  // meet 16 different bank groups (ordered by column they met four).
+  // Accumulator f, element e: row 4 * (lane / 16) + e, column CPL c + f, in column
+  // order (a lane with `extra` swaps its halves: the neighbour's columns land where
+  // none exist).  An order that spreads a write's 16 lanes over the LDS banks makes
+  // the partials' stores below strided, and lost more there: 16 x 12288, K 4096, 13.1
+  // us against 12.9; 16 x 10304, K 8640, 20.2 against 19.9.  Rows past M are written
+  // too: a branch around them takes longer (13.7 at 16 x 12288).
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (4 * kg + e < M)
 #pragma unroll
-      for (int f = 0; f < CPL; f += 4)
-        if (f >= extra)
-          *reinterpret_cast<f32x4d*>(&part[wave][(4 * kg + e) * DEC_COLS + ((f - extra) * 4 + c) * 4]) =
-              f32x4d{acc[f][e], acc[f + 1][e], acc[f + 2][e], acc[f + 3][e]};
+    for (int f = 0; f < CPL; f += 4)
+      *reinterpret_cast<f32x4d*>(&part[wave][(4 * kg + e) * DEC_COLS + c * CPL + (f ^ extra)]) =
+          f32x4d{acc[f][e], acc[f + 1][e], acc[f + 2][e], acc[f + 3][e]};
   __syncthreads();
   // Fixed-order sum of the eight wave partials; thread t owns the float4 chunks
   // t and t + 512 of the tile (the first only at 128 columns).
@@ -314,7 +315,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
   }
   auto store_y = [&](int q, f32x4d v) {
     const int i = (threadIdx.x + q * DEC_THREADS) * 4;
-    const int m = i / DEC_COLS, ch = i % DEC_COLS / 4, cc = ch % 16 * CPL + ch / 16 * 4;
+    const int m = i / DEC_COLS, cc = i % DEC_COLS;
     if (m < M && cc < ncols) {  // ncols % 8 == 0, so a chunk is all in or all out
       u32x2 h;
       h[0] = as_u32(f16x2{(_Float16)v[0], (_Float16)v[1]});
@@ -345,7 +346,7 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
   const rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(partials, 0, 0x7FFFFFFF, (int)RSRC_DW3);
   auto poff = [&](int s2, int q) -> uint32_t {
     const int i = (threadIdx.x + q * DEC_THREADS) * 4;
-    const int m = i / DEC_COLS, ch = i % DEC_COLS / 4, cc = ch % 16 * CPL + ch / 16 * 4;
+    const int m = i / DEC_COLS, cc = i % DEC_COLS;
     return (m < M && cc < ncols) ? (uint32_t)((((int64_t)s2 * M + m) * N + n0 + cc) * 4) : OOB;
   };
 #pragma unroll
