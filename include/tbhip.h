@@ -237,7 +237,12 @@ tb_status tb_fused_moe_w4a16(const uint16_t* X, const float* logits, const uint8
 /*
  * Row/column-scaled fp8 GEMM (step 2):
  *   Y bf16 [M, N] = bf16(sa[m] * sw[n] * sum_k e4m3(Aq[m,k]) * e4m3(Wq[k,n])),
- *   fp32 accumulation on the e4m3 matrix cores, one RNE rounding.
+ *   fp32 accumulation on the e4m3 matrix cores, one RNE rounding.  Results are
+ *   reproducible bit for bit.  The sum over K has one order, whatever M and N,
+ *   except on the 32 x 32 tiles that some calls of few rows take (chosen by M, N and K:
+ *   tb_gemm_tile's fp8_skinny), where four contiguous parts of K are summed and added
+ *   in order: there a row's last bf16 bit may differ from the same row's in a
+ *   larger call.
  *   Aq uint8 [M, K] row-major; WqT uint8 [N, K] row-major (the K-contiguous
  *   "column-major" weight layout); sa fp32 [M]; sw fp32 [N].
  * Requires K % 128 == 0, N % 8 == 0, each operand < 2 GiB, Aq / WqT / Y
@@ -261,8 +266,13 @@ tb_status tb_fp8_scaled_gemm(const uint8_t* Aq, const uint8_t* WqT, const float*
  *   and Aq 8-byte aligned.
  * tb_fp8_block_gemm: Y bf16 [M, N] =
  *   bf16( sum_kb (sa[kb, m] * sw[n/128, kb]) * sum_{k in block kb} Aq[m,k] * WqT[n,k] ),
- *   the block sums in fp32 on the e4m3 matrix cores, scaled and added in fp32
- *   in block order, one RNE rounding.  WqT uint8 [N, K]; sw fp32
+ *   the block sums in fp32 on the e4m3 matrix cores, scaled and added in fp32, one
+ *   RNE rounding.  Results are reproducible bit for bit.  The blocks are added in
+ *   block order, except on tiles whose wavefronts share K (chosen by M, N and K; tb_gemm_tile
+ *   reports k_groups > 1): with two groups the even and the odd blocks are added
+ *   separately, in order, and then the two sums; with four (32 x 32 tiles) four contiguous
+ *   ranges of blocks, then their sums in order.  A row's last bf16 bit may so differ
+ *   between calls of different M.  WqT uint8 [N, K]; sw fp32
  *   [ceil(N/128), K/128] row-major.  Requires K % 128 == 0, K <= 65536,
  *   N % 8 == 0, each operand < 2 GiB, Aq, WqT and Y 16-byte aligned.
  * Replace: the reference's block-scaled weight dequantisation

@@ -193,6 +193,41 @@ def test_fp8_tiles_match_oracle(gpu, tile, scaling):
         assert torch.equal(Y.view(torch.int16), again.view(torch.int16))
 
 
+@pytest.mark.parametrize("scaling", ["row", "block"])
+def test_fp8_rows_across_tiles(gpu, scaling):
+    """The first M rows of a call alone, against the same rows on 256 x 256 tiles:
+    equal bits wherever one wavefront group adds all of K, and otherwise a bf16 step
+    of rounding beside the fp32 sums' own error (9 blocks, each sum at most 9 max |y|)."""
+    N, K = 8200, 1152
+    if scaling == "row":
+        from tilebench_amd.benchmarks.operators.fp8_scaled_gemm import impl_hip
+        gen, op = T.generate_fp8_scaled_gemm_inputs, rt.OP_FP8_SCALED
+    else:
+        from tilebench_amd.benchmarks.operators.fp8_block_scaled_gemm import impl_hip
+        gen, op = T.generate_fp8_block_scaled_gemm_inputs, rt.OP_FP8_BLOCK
+    Aq, W, sa, sw = (t.to(gpu) for t in gen(1024, N, K, seed=11, device="cpu"))
+    WT = W.t().contiguous() if scaling == "row" else W
+    big = impl_hip.run(Aq, W, sa, sw)
+    assert rt.gemm_tile(op, 1024, N, K)["BM"] == 256
+    groups = set()
+    for M, n in [(16, 2112), (64, N), (192, N), (300, N), (448, N), (512, N)]:
+        t = rt.gemm_tile(op, M, n, K)
+        _say("fp8 rows", scaling, M, n, K, t)
+        w = WT[:n].contiguous()
+        s = sa[:M].contiguous() if scaling == "row" else sa[:, :M].contiguous()
+        got = impl_hip.run(Aq[:M].contiguous(), w.t() if scaling == "row" else w, s,
+                           sw[:n].contiguous() if scaling == "row" else sw[:-(-n // 128)].contiguous())
+        want = big[:M, :n]
+        torch.cuda.synchronize()
+        groups.add((t["kernel"], t["k_groups"]))
+        if t["k_groups"] == 1:
+            assert torch.equal(got.view(torch.int16), want.contiguous().view(torch.int16))
+        else:
+            d, y = (got.double() - want.double()).abs(), want.double().abs()
+            assert bool((d <= 2.0 ** -7 * y + 9 * 9 * 2.0 ** -24 * y.max()).all())
+    assert groups == {("fp8_skinny", 4), ("fp8_tile", 1)} | ({("fp8_tile", 2)} if scaling == "block" else set())
+
+
 @pytest.mark.parametrize("tile", list(NT_TILES))
 @pytest.mark.parametrize("dt", ["fp16", "fp32", "fp8", "int8"])
 def test_plain_product_tiles_match_oracle(gpu, tile, dt):

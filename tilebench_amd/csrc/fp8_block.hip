@@ -9,8 +9,9 @@
 //                             block-major ([K/128, M], M contiguous).
 //   tb_fp8_block_gemm         Y[m, n] = bf16( sum_kb (sa[kb, m] * sw[n/128, kb]) * P_kb[m, n] ),
 //                             P_kb = sum_{k in block kb} Aq[m,k] * WqT[n,k] in fp32 on the
-//                             fp8 matrix cores; the scaled block sums are added in fp32
-//                             in block order.  sw is the checkpoint's weight_scale_inv
+//                             fp8 matrix cores; the scaled block sums are added in fp32,
+//                             here in block order (fp8_small.hip, which takes calls of
+//                             few 256 x 256 tiles, may add parts of K apart).  sw is the checkpoint's weight_scale_inv
 //                             layout, [ceil(N/128), K/128] row-major.
 //
 // GEMM structure.  One 256 x 256 output tile per 512-thread block: eight

@@ -20,7 +20,9 @@
 //           rounded once to bf16.
 // fp8_tile, the rest, shares both operands through LDS (see there).
 // Block scales: P = the step's MFMAs from zero, acc += (sa * sw) * P in fp32 (one
-// FMA per element), in block order (in fp8_skinny within a wavefront's range).
+// FMA per element), in block order within a K group: a wavefront's contiguous range in
+// fp8_skinny, the even or the odd steps in fp8_tile with two groups, all of K otherwise.
+// fp8_tile without K groups gives the 256 x 256 kernels' bits.
 #include "fp8_small.h"
 
 #include "tb_common.h"
