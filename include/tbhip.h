@@ -101,9 +101,10 @@ tb_status tb_fp8_act_quant(const uint16_t* A, uint8_t* Aq, float* sa, int64_t M,
  * allocated: the kernel leaves its counters at zero after every call, so one
  * workspace serves consecutive calls on one stream; calls that overlap in time
  * must not share a workspace).  Larger M runs the MFMA prefill kernel and
- * needs no workspace; a row's result does not depend on the other rows, except
- * that up to 64 rows the fp32 sums over K are added in another order (four
- * groups), reproducibly.
+ * needs no workspace; there a row's result does not depend on the other rows,
+ * except that calls of up to 64 rows may add the fp32 sums over K in another
+ * order, four groups (all but those of wide N, where one order fills the
+ * device: tb_gemm_tile reports k_groups), reproducibly.
  * Replaces: matmul_fp32_fp16_fp8/impl_triton.py:124 run(a, b) (the reference's
  * fp16 GEMM operator), with the weight operand kept int4 in HBM.
  */
@@ -165,8 +166,9 @@ tb_status tb_w4a16_gemm_noalloc(const uint16_t* A, const uint8_t* W, const uint1
  *   A fp16 [R, K]; W uint8 [E, K, N/2]; scales fp16 [E, K/G, N];
  *   zeros uint8 [E, K/G, N/2]; offsets int32 [E+1] in device memory,
  *   non-decreasing from 0 to R -> Y fp16 [R, N] (rows outside every segment are
- *   left untouched).  Each expert's product is exactly tb_w4a16_gemm's for more
- *   than 64 rows (below, that call adds the sums over K in another order).
+ *   left untouched).  Each expert's product has the bits of tb_w4a16_gemm for
+ *   more than 64 rows, however many rows the expert has (below, that call may
+ *   add the sums over K in another order).
  * Requires N % 8 == 0, K % 64 == 0, G % 64 == 0, K % G == 0, E <= 4096,
  * A < 4 GiB, one expert's W < 2 GiB; A, scales, Y 16-byte aligned.
  * Replaces: no reference operator (the reference has no grouped GEMM); the

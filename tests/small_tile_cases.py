@@ -16,8 +16,9 @@ EXPERT_TILE_IDS = {"256": 0, "32x128": 1, "32x256": 2, "64x256": 3}
 #: fewer steps than K groups, N % 32 != 0
 DENSE_TILES = {
     "64x64": [(17, 64, 8, 64), (33, 320, 392, 64), (64, 704, 1000, 64), (48, 2048, 4096, 128)],
-    "64x128": [(65, 64, 264, 64), (129, 448, 1096, 64), (500, 192, 4096, 64)],
-    "64x256": [(300, 192, 22040, 64), (1000, 128, 4096, 64)],
+    # up to 64 rows too where N alone fills the device
+    "64x128": [(65, 64, 264, 64), (129, 448, 1096, 64), (500, 192, 4096, 64), (64, 64, 32768, 64)],
+    "64x256": [(300, 192, 22040, 64), (1000, 128, 4096, 64), (40, 64, 65536, 64)],
     "128x256": [(768, 320, 8944, 64), (2047, 64, 4096, 64)],
     # half a round and more of 256 x 256 tiles: two rounds and a bit of a smaller tile take 20 - 28 % longer
     "256": [(1024, 192, 11008, 64), (691, 192, 11896, 64), (729, 64, 12288, 64), (1725, 64, 5480, 64),

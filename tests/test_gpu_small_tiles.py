@@ -115,10 +115,11 @@ def test_dense_tiles_match_oracle(gpu, tile):
                                    rtol=1e-2)
 
 
-@pytest.mark.parametrize("M,N,tile", [(65, 11008, (64, 128)), (500, 11008, (128, 256)), (300, 22040, (64, 256))])
+@pytest.mark.parametrize("M,N,tile", [(65, 11008, (64, 128)), (500, 11008, (128, 256)), (300, 22040, (64, 256)),
+                                      (64, 32768, (64, 128))])
 def test_dense_rows_do_not_depend_on_the_tile(gpu, M, N, tile):
-    """More than 64 rows: the first M rows alone give the bits they have in a
-    product of 256 x 256 tiles.  64 rows (K in four groups) are reproducible."""
+    """Tiles that do not split K: the first M rows alone give the bits they have in a
+    product of 256 x 256 tiles, at 64 rows too where N is wide.  64 rows are reproducible."""
     from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
 
     A, p, s, z, G = T.generate_w4a16_gemm_inputs(1024, 448, N, 64, seed=3, device="cpu")

@@ -27,9 +27,10 @@
 // dequantisation to fp16, the same v_mfma_f32_32x32x16_f16 operands in the same
 // K order per output element, the same epilogue roundings; results are
 // bit-identical to them, so neither the choice of tile nor the call that uses
-// it shows in an output.  Only the dense product of at most 64 rows (S32x64k4, S64x64k4)
-// splits K, over four groups of wavefronts of one block whose fp32 sums are
-// added through LDS in group order: reproducible, but not the unsplit order.
+// it shows in an output.  Only the 64-column dense tiles (S32x64k4, S64x64k4), which take
+// products of at most 64 rows unless N alone fills the device with wider ones,
+// split K, over four groups of wavefronts of one block whose fp32 sums are added
+// through LDS in group order: reproducible, but not the unsplit order.
 // No workspace is needed.
 #include "w4a16_small.h"
 
@@ -70,7 +71,8 @@ struct Shape {
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
 
-// The shapes in use (three stages: four measured the same, two 10 - 30 % slower).
+// The shapes in use.  Three stages (four measured the same, two 10 - 30 % slower); four
+// at 64 x 128, where three blocks of 51 KiB still share a CU.
 typedef Shape<1, 2, true, 1, 3> S32x128;
 typedef Shape<1, 4, false, 1, 3> S32x256;
 typedef Shape<2, 4, false, 1, 3> S64x256;
