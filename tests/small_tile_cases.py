@@ -10,6 +10,21 @@ EXPERT_TILES = {
     "64x256": [([63, 64, 65, 1, 0, 129, 128, 40] * 8, 1408, 192, 64), ([100] * 33, 2056, 320, 64)],
     "256": [([600, 511, 700, 0, 512, 513, 900, 255] * 8, 1408, 128, 64)],
 }
+#: (tile, 16-byte weight loads) -> (tokens, experts, top k, K, columns, group) of the gate/up
+#: (columns I: 16-byte loads where I % 32 == 0) and down products (columns H, likewise):
+#: tokens routed nowhere, an expert without rows or with several row tiles, ragged last column tiles
+GATE_UP_TILES = {
+    ("32x128", True): (33, 5, 3, 320, 96, 64), ("32x128", False): (33, 5, 3, 320, 72, 64),
+    ("32x256", True): (70, 70, 2, 192, 704, 64), ("32x256", False): (70, 70, 2, 128, 712, 128),
+    ("64x256", True): (500, 32, 4, 128, 704, 64), ("64x256", False): (500, 32, 4, 192, 712, 64),
+    ("256", True): (1500, 16, 4, 128, 704, 64), ("256", False): (1500, 16, 4, 64, 712, 64),
+}
+DOWN_TILES = {
+    ("32x128", True): (33, 5, 3, 192, 320, 64), ("32x128", False): (33, 5, 3, 64, 328, 64),
+    ("32x256", True): (24, 64, 8, 192, 1408, 64), ("32x256", False): (70, 70, 2, 128, 1416, 128),
+    ("64x256", True): (500, 32, 4, 192, 1408, 64), ("64x256", False): (500, 32, 4, 64, 1416, 64),
+    ("256", True): (1500, 16, 4, 128, 1408, 64), ("256", False): (1500, 16, 4, 64, 1416, 64),
+}
 EXPERT_TILE_IDS = {"256": 0, "32x128": 1, "32x256": 2, "64x256": 3}
 
 #: tile -> (M, K, N, group) of the dense product: ragged rows and columns, K of

@@ -7,7 +7,8 @@ import pytest
 import torch
 
 import oracle
-from small_tile_cases import DECODE_PLANS, DENSE_TILES, EXPERT_TILES, FP8_TILES, NT_TILES
+from small_tile_cases import (DECODE_PLANS, DENSE_TILES, DOWN_TILES, EXPERT_TILES, FP8_TILES, GATE_UP_TILES,
+                              NT_TILES)
 from tilebench_amd import runtime as rt
 from tilebench_amd.data import tensors as T
 
@@ -39,9 +40,9 @@ def test_grouped_tiles_match_oracle(gpu, tile):
         np.testing.assert_allclose(Y.cpu().numpy().astype(np.float32), ref.astype(np.float32), atol=1e-2, rtol=1e-2)
 
 
-@pytest.mark.parametrize("per_expert", [1, 20, 60])  # 32 x 128 (one column), 32 x 256 and 64 x 256 tiles
-def test_grouped_rows_do_not_depend_on_the_tile(gpu, per_expert):
-    """The first rows of every expert alone give the bits they have in a call
+@pytest.mark.parametrize("per_expert,experts,tile", [(1, 8, (32, 128)), (20, 64, (32, 256)), (60, 64, (64, 256))])
+def test_grouped_rows_do_not_depend_on_the_tile(gpu, per_expert, experts, tile):
+    """The first rows of the first experts alone give the bits they have in a call
     whose experts fill 256-row tiles."""
     from tilebench_amd.benchmarks.operators.moe_w4a16_grouped_gemm import impl_hip
 
@@ -50,7 +51,10 @@ def test_grouped_rows_do_not_depend_on_the_tile(gpu, per_expert):
     A, p, s, z, off = _grouped(rows, N, K, G, seed=5)
     d = [t.to(gpu) for t in (A, p, s, z)]
     big = impl_hip.run(*d, off.to(gpu), G)
-    take = [min(r, per_expert) for r in rows]
+    take = [min(r, per_expert) if e < experts else 0 for e, r in enumerate(rows)]
+    for n, t in ((sum(take), tile), (sum(rows), (256, 256))):
+        picked = rt.gemm_tile(rt.OP_W4A16_GROUPED, n, N, K, len(rows))
+        assert (picked["BM"], picked["BN"]) == t
     o2 = torch.zeros(len(rows) + 1, dtype=torch.int32)
     o2[1:] = torch.cumsum(torch.tensor(take), 0)
     idx = torch.cat([torch.arange(int(off[e]), int(off[e]) + n) for e, n in enumerate(take)]).to(gpu)
@@ -62,9 +66,9 @@ def test_grouped_rows_do_not_depend_on_the_tile(gpu, per_expert):
 @pytest.mark.parametrize("Tk,E,k,H,I,g", [(1, 8, 4, 256, 128, 64), (33, 5, 3, 320, 72, 64), (70, 70, 2, 192, 704, 64),
                                           (500, 16, 8, 128, 704, 64), (700, 16, 8, 192, 1032, 64)])
 def test_gate_up_and_down_tiles_match_oracle(gpu, Tk, E, k, H, I, g):
-    """Token gather, SiLU epilogue, routing weights and the scatter on each
-    tile; I % 32 != 0 and H % 32 != 0 take the 4-byte weight loads.  Pairs
-    routed nowhere stay unwritten."""
+    """Token gather, SiLU epilogue, routing weights and the scatter, the down
+    product on the gate/up product's rows, where the two take different tiles
+    too.  Pairs routed nowhere stay unwritten."""
     _say("gate_up + down", Tk, E, k, H, I, g)
     gen = T._gen(Tk + I)
     X = torch.randn(Tk, H, generator=gen).to(torch.float16)
@@ -95,6 +99,54 @@ def test_gate_up_and_down_tiles_match_oracle(gpu, Tk, E, k, H, I, g):
             *map(rt.ptr, d2), rt.ptr(y), P, E, I, H, 64, rt.stream_handle(gpu))
     torch.cuda.synchronize()
     want, written = oracle.moe_down(got, sid, off, w.numpy(), P, *(t.numpy() for t in W2), 64)
+    y = y.cpu().numpy()
+    np.testing.assert_allclose(y[written].astype(np.float32), want[written].astype(np.float32), atol=1e-2, rtol=1e-2)
+    assert np.isnan(y[~written].astype(np.float32)).all()
+
+
+def _routed(T_, E, k, gen, gpu):
+    """(ids by expert, offsets, routing weights) on the host and on the GPU; every fifth token's first pair goes nowhere."""
+    ids = T.zipf_routing(T_, k, E, 1.1, seed=7).to(torch.int32)
+    ids[::5, 0] = E + 2
+    w = torch.rand(T_, k, generator=gen)
+    sid, off = oracle.moe_align(ids.numpy(), E)
+    sorted_ids = np.full(T_ * k, -1, np.int32)
+    sorted_ids[:len(sid)] = sid
+    return sid, off, w, [t.to(gpu) for t in (torch.from_numpy(sorted_ids), torch.from_numpy(off), w)]
+
+
+@pytest.mark.parametrize("tile,wide", list(GATE_UP_TILES))
+def test_gate_up_tiles_match_oracle(gpu, tile, wide):
+    Tk, E, k, H, I, g = GATE_UP_TILES[tile, wide]
+    _say("gate_up", tile, wide, Tk, E, k, H, I, g)
+    gen = T._gen(Tk + I)
+    X = torch.randn(Tk, H, generator=gen).to(torch.float16)
+    sid, off, _, (dsid, doff, _) = _routed(Tk, E, k, gen, gpu)
+    W = T.random_int4_weights(H, 2 * I, g, gen, experts=E)
+    dX, dW = X.to(gpu), [t.to(gpu) for t in W]
+    act = torch.empty((Tk * k, I), dtype=torch.float16, device=gpu)
+    rt.call("tb_moe_w4a16_gate_up", rt.ptr(dX), rt.ptr(dsid), rt.ptr(doff), *map(rt.ptr, dW), rt.ptr(act), Tk, k, E, H, I,
+            g, rt.stream_handle(gpu))
+    torch.cuda.synchronize()
+    want = oracle.moe_gate_up(X.numpy(), sid, off, k, *(t.numpy() for t in W), g)[:len(sid)]
+    np.testing.assert_allclose(act.cpu().numpy()[:len(sid)].astype(np.float32), want.astype(np.float32), atol=1e-2,
+                               rtol=1e-2)
+
+
+@pytest.mark.parametrize("tile,wide", list(DOWN_TILES))
+def test_down_tiles_match_oracle(gpu, tile, wide):
+    Tk, E, k, I, H, g = DOWN_TILES[tile, wide]
+    _say("down", tile, wide, Tk, E, k, I, H, g)
+    gen = T._gen(Tk + H)
+    act = torch.randn(Tk * k, I, generator=gen).to(torch.float16)
+    sid, off, w, (dsid, doff, dw) = _routed(Tk, E, k, gen, gpu)
+    W = T.random_int4_weights(I, H, g, gen, experts=E)
+    dact, dW = act.to(gpu), [t.to(gpu) for t in W]
+    y = torch.full((Tk * k, H), float("nan"), dtype=torch.float16, device=gpu)
+    rt.call("tb_moe_w4a16_down", rt.ptr(dact), rt.ptr(dsid), rt.ptr(doff), rt.ptr(dw), *map(rt.ptr, dW), rt.ptr(y), Tk * k,
+            E, I, H, g, rt.stream_handle(gpu))
+    torch.cuda.synchronize()
+    want, written = oracle.moe_down(act.numpy(), sid, off, w.numpy(), Tk * k, *(t.numpy() for t in W), g)
     y = y.cpu().numpy()
     np.testing.assert_allclose(y[written].astype(np.float32), want[written].astype(np.float32), atol=1e-2, rtol=1e-2)
     assert np.isnan(y[~written].astype(np.float32)).all()

@@ -6,7 +6,8 @@ import subprocess
 
 import pytest
 
-from small_tile_cases import DECODE_PLANS, DENSE_TILE_IDS, DENSE_TILES, EXPERT_TILE_IDS, EXPERT_TILES, FP8_TILE_IDS, FP8_TILES, NT_TILE_IDS, NT_TILES
+from small_tile_cases import (DECODE_PLANS, DENSE_TILE_IDS, DENSE_TILES, DOWN_TILES, EXPERT_TILE_IDS, EXPERT_TILES,
+                              FP8_TILE_IDS, FP8_TILES, GATE_UP_TILES, NT_TILE_IDS, NT_TILES)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -26,6 +27,17 @@ def test_expert_tiles_picked(tmp_path):
     args = [str(x) for _, *c in cases for x in c]
     got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
     assert [int(g) for g in got] == [EXPERT_TILE_IDS[c[0]] for c in cases]
+
+
+def test_gate_up_and_down_tiles_picked(tmp_path):
+    """Each tile once with 16-byte and once with 4-byte weight loads."""
+    exe = _build(tmp_path)
+    for cases, columns in ((GATE_UP_TILES, 2), (DOWN_TILES, 1)):
+        assert set(cases) == {(t, w) for t in EXPERT_TILE_IDS for w in (True, False)}
+        args = [str(x) for T, E, k, _, n, _ in cases.values() for x in (T * k, E, columns * n)]
+        got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
+        assert [int(g) for g in got] == [EXPERT_TILE_IDS[t] for t, _ in cases]
+        assert [n % 32 == 0 for *_, n, _ in cases.values()] == [w for _, w in cases]
 
 
 def test_dense_tiles_picked(tmp_path):
