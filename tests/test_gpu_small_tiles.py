@@ -389,3 +389,129 @@ def test_config_names_what_was_launched(gpu, op, case):
             assert cfg["tile"] == f"{args[2]}x{args[3]}"
         else:
             assert kernel == "fp8_skinny" and (cfg["BM"], cfg["BN"], cfg["waves"]) == (32, 32, args[0])
+
+
+def _same_specials(got, want):
+    """NaN and infinities (with their signs) of `got` where `want` has them."""
+    got, want = got.double().cpu(), want.double().cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(got.isinf(), inf) and torch.equal(got[inf], want[inf])
+
+
+@pytest.mark.parametrize("tile", ["32x32", "64x64", "64x128", "128x128"])
+@pytest.mark.parametrize("scaling", ["row", "block"])
+def test_fp8_special_rows(gpu, tile, scaling):
+    """Row 0 as the quantiser leaves a row of zeros (scale 0, NaN codes), row 2 of
+    infinite scale, row 5 with one NaN code: their own outputs as IEEE has them, and
+    every other row's bits as without them."""
+    if scaling == "row":
+        from tilebench_amd.benchmarks.operators.fp8_scaled_gemm import impl_hip
+        gen = T.generate_fp8_scaled_gemm_inputs
+    else:
+        from tilebench_amd.benchmarks.operators.fp8_block_scaled_gemm import impl_hip
+        gen = T.generate_fp8_block_scaled_gemm_inputs
+    M, N, K = next(c for c in FP8_TILES[tile] if c[0] > 8)
+    _say("fp8 special rows", scaling, tile, M, N, K)
+    Aq, W, sa, sw = (t.to(gpu) for t in gen(M, N, K, seed=M, device="cpu"))
+    plain = impl_hip.run(Aq, W, sa, sw)
+    codes, scale = Aq.view(torch.uint8).clone(), sa.clone()
+    rows = scale if scaling == "row" else scale.t()  # [M] or [M, K / 128], views
+    codes[0], codes[5, K - 1] = 0xFF, 0x7F
+    rows[0], rows[2] = 0.0, float("inf")
+    Y = impl_hip.run(codes.view(torch.float8_e4m3fn), W, scale, sw)
+    torch.cuda.synchronize()
+    others = [m for m in range(M) if m not in (0, 2, 5)]
+    assert torch.equal(Y[others].view(torch.int16), plain[others].view(torch.int16))
+    assert bool(Y[[0, 5]].isnan().all())
+    if scaling == "row":  # one product, then the scale: +-inf, as the plain row's signs
+        _same_specials(Y[2], plain[2].float() * float("inf"))
+    else:  # infinite terms of either sign: NaN unless K has one block
+        assert not bool(Y[2].isfinite().any())
+
+
+@pytest.mark.parametrize("tile", ["64x64", "64x128", "64x256", "128x256"])
+def test_dense_special_rows(gpu, tile):
+    """A row of NaN, one infinity and a row of the largest values: their own outputs
+    as the oracle has them, and every other row's bits as without them."""
+    from tilebench_amd.benchmarks.operators.w4a16_gemm import impl_hip
+
+    M, K, N, G = DENSE_TILES[tile][1]
+    _say("dense special rows", tile, M, K, N, G)
+    A, p, s, z, G = T.generate_w4a16_gemm_inputs(M, K, N, G, seed=M, device="cpu")
+    d = [t.to(gpu) for t in (p, s, z)]
+    plain = impl_hip.run(A.to(gpu), *d, G)
+    B = A.clone()
+    B[1], B[3, K - 1], B[M - 1] = float("nan"), float("-inf"), 65504.0
+    Y = impl_hip.run(B.to(gpu), *d, G)
+    torch.cuda.synchronize()
+    others = [m for m in range(M) if m not in (1, 3, M - 1)]
+    assert torch.equal(Y[others].view(torch.int16), plain[others].view(torch.int16))
+    rows = [1, 3, M - 1]
+    with np.errstate(all="ignore"):
+        want = torch.from_numpy(oracle.w4a16_gemm(B.numpy()[rows], p.numpy(), s.numpy(), z.numpy(), G))
+    _same_specials(Y[rows[:2]], want[:2])
+    # sums of 65504 w near fp16's own largest value may round to infinity in one order and not in another
+    clear = (want[2].float().abs() < 6e4) | want[2].isinf()
+    got = Y[M - 1].cpu()
+    big = want[2].isinf() & got.isinf()
+    assert torch.equal(got[big], want[2][big]) and not bool(got.isnan().any())
+    assert bool((got[clear & ~want[2].isinf()].isfinite()).all())
+
+
+@pytest.mark.parametrize("tile", ["64x64", "64x128", "128x128"])
+@pytest.mark.parametrize("dt", ["fp16", "fp8"])
+def test_plain_product_special_rows(gpu, tile, dt):
+    from tilebench_amd.benchmarks.operators.matmul_fp32_fp16_fp8 import impl_hip
+
+    M, N, Kb = NT_TILES[tile][-1] if tile != "128x128" else NT_TILES[tile][0]
+    K = Kb // 2 if dt == "fp16" else Kb
+    _say("plain special rows", dt, tile, M, N, K)
+    tdt = torch.float16 if dt == "fp16" else torch.float8_e4m3fn
+    a, b = (t.to(gpu) for t in T.generate_matmul_fp32_fp16_fp8_inputs(M, N, K, dtype=tdt, seed=M, device="cpu"))
+    plain = impl_hip.run(a, b)
+    c = a.clone()
+    raw = c.view(torch.uint8 if dt == "fp8" else torch.int16)
+    nan, other = (0x7F, 0xFF) if dt == "fp8" else (0x7E00, 0x7C00)  # fp8 has no infinity: the other NaN code
+    raw[1], raw[4, K - 1] = nan, other
+    Y = impl_hip.run(c, b)
+    torch.cuda.synchronize()
+    others = [m for m in range(M) if m not in (1, 4)]
+    bits = torch.uint8 if dt == "fp8" else torch.int16
+    assert torch.equal(Y[others].view(bits), plain[others].view(bits))
+    assert bool(Y[1].float().isnan().all())
+    if dt == "fp8":
+        assert bool(Y[4].float().isnan().all())
+    else:
+        _same_specials(Y[4], float("inf") * b[K - 1].float())  # inf times 0 is NaN
+
+
+@pytest.mark.parametrize("M,N,tile", [(64, 136, (64, 64)), (320, 4104, (64, 128)), (640, 4104, (128, 128))])
+def test_fp8_block_scales_at_the_largest_k(gpu, M, N, tile):
+    """K = 65536: 512 scale blocks fill the tiles' scale table.  The last rows and
+    columns against 64-bit sums; fp32 sums of 512 blocks, then bf16 (half a step, 2^-9)."""
+    from tilebench_amd.benchmarks.operators.fp8_block_scaled_gemm import impl_hip
+
+    K = 65536
+    t = rt.gemm_tile(rt.OP_FP8_BLOCK, M, N, K)
+    assert (t["BM"], t["BN"]) == tile
+    _say("fp8 block, largest K", M, N, t)
+    g = torch.Generator(device=gpu).manual_seed(M)
+    Aq, W = ((torch.randint(0, 112, (n, K), generator=g, device=gpu, dtype=torch.uint8)
+              | torch.randint(0, 2, (n, K), generator=g, device=gpu, dtype=torch.uint8) << 7).view(torch.float8_e4m3fn)
+             for n in (M, N))  # both signs, at most 120
+    sa = torch.rand(K // 128, M, generator=g, device=gpu) + 0.5
+    sw = torch.rand(-(-N // 128), K // 128, generator=g, device=gpu) + 0.5
+    Y = impl_hip.run(Aq, W, sa, sw)
+    r, c = slice(max(0, M - 32), M), slice(max(0, N - 64), N)
+    a = Aq[r].float().double().view(-1, K // 128, 128) * sa[:, r].t().double()[:, :, None]
+    scale = sw.double().repeat_interleave(128, dim=0)[:N][c]
+    w = W[c].float().double().view(-1, K // 128, 128) * scale[:, :, None]
+    want, size = torch.zeros_like(Y[r, c], dtype=torch.float64), torch.zeros_like(Y[r, c], dtype=torch.float64)
+    for kb in range(K // 128):
+        want += a[:, kb] @ w[:, kb].t()
+        size += a[:, kb].abs() @ w[:, kb].abs().t()
+    torch.cuda.synchronize()
+    # 128-term and 512-term fp32 sums: (128 + 512) roundings of 2^-24 of the sum of magnitudes at most
+    bound = 2.0 ** -8 * want.abs() + 640 * 2.0 ** -24 * size
+    assert bool(((Y[r, c].double() - want).abs() <= bound).all())
