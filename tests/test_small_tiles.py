@@ -21,12 +21,17 @@ def _build(tmp_path):
     return exe
 
 
+def _picks(exe, groups):
+    """The numbers that each (rule, a, b, c) prints."""
+    args = [str(x) for g in groups for x in g]
+    out = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout
+    return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+
 def test_expert_tiles_picked(tmp_path):
-    exe = _build(tmp_path)
     cases = [(tile, sum(rows), len(rows), N) for tile, cs in EXPERT_TILES.items() for rows, N, _, _ in cs]
-    args = [str(x) for _, *c in cases for x in c]
-    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-    assert [int(g) for g in got] == [EXPERT_TILE_IDS[c[0]] for c in cases]
+    got = _picks(_build(tmp_path), [("expert", *c) for _, *c in cases])
+    assert [g for g, in got] == [EXPERT_TILE_IDS[c[0]] for c in cases]
 
 
 def test_gate_up_and_down_tiles_picked(tmp_path):
@@ -34,54 +39,41 @@ def test_gate_up_and_down_tiles_picked(tmp_path):
     exe = _build(tmp_path)
     for cases, columns in ((GATE_UP_TILES, 2), (DOWN_TILES, 1)):
         assert set(cases) == {(t, w) for t in EXPERT_TILE_IDS for w in (True, False)}
-        args = [str(x) for T, E, k, _, n, _ in cases.values() for x in (T * k, E, columns * n)]
-        got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-        assert [int(g) for g in got] == [EXPERT_TILE_IDS[t] for t, _ in cases]
+        got = _picks(exe, [("expert", T * k, E, columns * n) for T, E, k, _, n, _ in cases.values()])
+        assert [g for g, in got] == [EXPERT_TILE_IDS[t] for t, _ in cases]
         assert [n % 32 == 0 for *_, n, _ in cases.values()] == [w for _, w in cases]
 
 
 def test_dense_tiles_picked(tmp_path):
-    exe = _build(tmp_path)
-    cases = [(tile, M, 0, N) for tile, cs in DENSE_TILES.items() for M, _, N, _ in cs]
-    args = [str(x) for _, *c in cases for x in c]
-    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-    assert [int(g) for g in got] == [DENSE_TILE_IDS[c[0]] for c in cases]
+    cases = [(tile, M, N) for tile, cs in DENSE_TILES.items() for M, _, N, _ in cs]
+    got = _picks(_build(tmp_path), [("dense", M, N, 0) for _, M, N in cases])
+    assert [g for g, in got] == [DENSE_TILE_IDS[c[0]] for c in cases]
 
 
 def test_fp8_tiles_picked(tmp_path):
-    exe = _build(tmp_path)
-    cases = [(tile, M, -K - blk, N) for tile, cs in FP8_TILES.items() for M, N, K in cs for blk in (0, 1)]
-    args = [str(x) for _, *c in cases for x in c]
-    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-    assert [int(g) for g in got] == [FP8_TILE_IDS[c[0]] for c in cases]
+    cases = [(tile, rule, *c) for tile, cs in FP8_TILES.items() for c in cs for rule in ("fp8", "fp8b")]
+    got = _picks(_build(tmp_path), [c for _, *c in cases])
+    assert [g for g, in got] == [FP8_TILE_IDS[c[0]] for c in cases]
 
 
 def test_plain_product_tiles_picked(tmp_path):
-    exe = _build(tmp_path)
-    cases = [(tile, M, -10 ** 9 - Kb, N) for tile, cs in NT_TILES.items() for M, N, Kb in cs]
-    args = [str(x) for _, *c in cases for x in c]
-    got = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-    assert [int(g) for g in got] == [NT_TILE_IDS[c[0]] for c in cases]
+    cases = [(tile, *c) for tile, cs in NT_TILES.items() for c in cs]
+    got = _picks(_build(tmp_path), [("nt", *c) for _, *c in cases])
+    assert [g for g, in got] == [NT_TILE_IDS[c[0]] for c in cases]
 
 
 def test_decode_plans_picked(tmp_path):
     """The listed plans, and for other sizes and CU counts the bounds that the
     kernel and its scratch rely on."""
     exe = _build(tmp_path)
-
-    def picks(cases):
-        args = [str(x) for cus, K, N in cases for x in (cus, -2 * 10 ** 9 - K, N)]
-        out = subprocess.run([exe, *args], check=True, capture_output=True, text=True).stdout.split()
-        return [(int(g) % 10 ** 9 // 1000, int(g) % 1000, int(g) // 10 ** 9) for g in out]
-
-    listed = [(plan, 256, K, N) for plan, cs in DECODE_PLANS.items() for N, K in cs]
-    assert [p[:2] for p in picks([c[1:] for c in listed])] == [c[0] for c in listed]
-    cases = [(cus, K, N) for cus in (1, 64, 256, 304) for K in (64, 192, 256, 1024, 7168, 32768)
+    listed = [(plan, N, K) for plan, cs in DECODE_PLANS.items() for N, K in cs]
+    assert [g[:2] for g in _picks(exe, [("decode", 256, N, K) for _, N, K in listed])] == [c[0] for c in listed]
+    cases = [(cus, N, K) for cus in (1, 64, 256, 304) for K in (64, 192, 256, 1024, 7168, 32768)
              for N in (8, 128, 1000, 4096, 32768, 32776, 65536)]
     # pairs of 128-column slabs that do not divide over the 8 XCDs: five splits of 26 pairs
     # would be 34 blocks on some XCDs of 32 CUs, three of 43 likewise
-    cases += [(256, 9920, 6528), (256, 4096, 10880), (256, 7744, 6448), (256, 2560, 10816), (256, 12672, 3136)]
-    for (cus, K, N), (cols, splits, blocks) in zip(cases, picks(cases)):
+    cases += [(256, 6528, 9920), (256, 10880, 4096), (256, 6448, 7744), (256, 10816, 2560), (256, 3136, 12672)]
+    for (cus, N, K), (cols, splits, blocks) in zip(cases, _picks(exe, [("decode", *c) for c in cases])):
         slabs = -(-N // cols)
         assert cols in (128, 256) and 1 <= splits <= 16
         assert splits == 1 or (slabs * splits <= cus and splits * 8 <= K // 32)
