@@ -69,9 +69,10 @@ NT_TILE_IDS = {"256": 0, "64x64": 1, "64x128": 2, "128x128": 3}
 #: shares of the units, half-filled 16-column lanes at 256 columns
 DECODE_PLANS = {
     (128, 1): [(8, 64), (136, 192), (2048, 1024), (264, 128)],
-    (128, 3): [(8944, 6080), (10112, 3200)],
+    (128, 3): [(9000, 3072), (10112, 3200)],
     (128, 4): [(1408, 4096), (4096, 4096), (5000, 3072)],
     (128, 8): [(4096, 11008)],
     (256, 1): [(32776, 1024)],
     (256, 5): [(12288, 4096), (12296, 4096)],
+    (256, 7): [(8944, 6080)],
 }

@@ -177,9 +177,14 @@ struct DecodePlan {
 // each at 128 columns and 1.45 at 256 (there a CU's stream binds: the mean share
 // counts, not the longest; K 4096, N 12288 from cold 14.1 on 192 CUs, 13.4 on 240); a
 // split costs an exchange of partials (1.5 or 3.6) that grows with the blocks taking
-// part (0.55 or 0.6 each); and 128-column slabs, which read half lines, lose 0.11 per
-// MB of weights.  Measured, 128 / 256 columns at their best splits: K 4096, N 4096
-// 7.8 / 11.4; K 4096, N 11008 11.4 / 12.5; K 4096, N 12288 13.5 / 13.2; K 8192, N
+// part (0.55 or 0.6 each); and 128-column slabs, which read half lines, lose 0.09 per
+// MB of weights and 0.2 more per MB above 23.  Fitted to 420 sizes, each with weights
+// that stay in the last-level cache, that rotate through HBM, and that follow a fill of
+// the cache with written lines: the picks take 0.2 - 0.3 % more than the better width, and 8
+// of 2520 take over 3 % more than the 256-column kernel that was here before (worst 1 x
+// 7184, K 6656, after a fill: 16.8 us against 15.3).  Measured, 128 / 256 columns at
+// their best splits: K 4096, N 4096
+// 7.8 / 11.4; K 4096, N 11008 11.9 / 12.5; K 4096, N 12288 14.4 / 12.9; K 8192, N
 // 28672 43.1 / 32.6.  Splits at 128
 // columns, K 4096, N 4096: 1 13.1, 2 9.7, 4 7.8, 8 8.5; K 1024, N 12288: 1 6.0, 2 6.7.
 // A split grid never has more blocks than CUs, counted as they are launched: pairs of
@@ -192,6 +197,7 @@ inline int64_t decode_grid(int cols, int64_t slabs, int splits) {
 
 inline DecodePlan pick_decode(int64_t N, int64_t K, int cus) {
   const int64_t units = K / DEC_UNIT;
+  const double mb = 0.5e-6 * (double)N * (double)K;  // of weights
   DecodePlan best{128, (N + 127) / 128, 1};
   double c = -1;
   for (int cols = 128; cols <= (N <= 128 ? 128 : 256); cols += 128) {  // the wide slab needs 16 columns
@@ -200,8 +206,8 @@ inline DecodePlan pick_decode(int64_t N, int64_t K, int cus) {
     for (int s = 1; s <= DEC_MAX_SPLITS && (s == 1 || (decode_grid(cols, slabs, s) <= cus && (int64_t)s * DEC_WAVES <= units)); ++s) {
       const double rounds = (double)((slabs * s + cus - 1) / cus), share = (double)units / (s * DEC_WAVES);
       double cost = wide ? rounds * std::max(1.0, share) * 1.45
-                         : rounds * (double)(int64_t)(share + 0.999999) * 0.75 + 0.055e-6 * (double)N * (double)K;
-      if (s > 1) cost += wide ? 3.6 + 0.6 * s : 1.5 + 0.55 * s;
+                         : rounds * (double)(int64_t)(share + 0.999999) * 0.75 + 0.09 * mb + 0.2 * std::max(0.0, mb - 23);
+      if (s > 1) cost += wide ? 3.6 + 0.6 * s : 2.1 + 0.55 * s;
       if (c < 0 || cost < c) best = DecodePlan{cols, slabs, s}, c = cost;
     }
   }

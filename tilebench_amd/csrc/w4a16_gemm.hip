@@ -179,9 +179,12 @@ __global__ void __launch_bounds__(DEC_THREADS, 2)
   const uint32_t a_off = arow < M ? ((uint32_t)arow * (uint32_t)K + (uint32_t)(kg * 8)) * 2u : OOB;
   const uint32_t s_off[2] = {col_ok ? (uint32_t)n * 2u : OOB, col_ok ? (uint32_t)(n + 8) * 2u : OOB};
   const uint32_t z_off[2] = {col_ok ? (uint32_t)(n >> 1) : OOB, col_ok ? (uint32_t)(n >> 1) + 4u : OOB};
-  // nontemporal where the weights are large and read once; not where the other half of
-  // the line is about to be read on the same XCD (172 blocks at M = 1 11.7 us, nontemporal 12.3)
-  constexpr int NT = WORDS == 1 ? 0 : 2;
+  // nontemporal: the weights are read once, and a read that allocates in the last-level
+  // cache first evicts what it holds.  16 x 11008 (K 4096), 128 columns, plain ->
+  // nontemporal: 17.9 -> 15.1 us after a fill of that cache with written lines (8192 x 8192
+  // 23.1 -> 18.2), 12.5 -> 11.9 on weights that rotate through HBM, 10.3 -> 10.9 on weights
+  // that stay in the cache.
+  constexpr int NT = 2;
 
   f32x4d acc[CPL];
 #pragma unroll
