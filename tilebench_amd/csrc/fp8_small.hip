@@ -449,12 +449,13 @@ tb_status launch_tile(const char* fn, const Fp8Args& a, hipStream_t stream) {
 
 // f(shape) of an LDS tile: launch and describe take the same one.
 // Ring stages: as deep as pays while one block runs per CU (64 x 64: four, 15.4
-// against 18.9 us with three at 64 x 8192 x 8192; 64 x 128: four, 14.0 against 15.0
-// at 512 x 4096 x 4096); two or three where several tiles share a CU, so that two
+// against 18.9 us with three at 64 x 8192 x 8192; 64 x 128: four, 11.9 against 13.1
+// at 300 x 5000 x 4096); two or three where several tiles share a CU, so that two
 // blocks fit (128 x 128: 1024 x 8192 x 8192 60 us with two, 70 with three).  With
 // block scales, one block per CU and one wavefront per SIMD, the scale FMAs wait for
-// the MFMAs; two K groups fill each other's waits (200 x 2112 x 7168 17.3 -> 13.8 us,
-// 128 x 8192 x 8192 20.6 -> 16.2, 300 x 5000 x 4096 14.4 -> 13.6; row scales: no gain).
+// the MFMAs; two K groups fill each other's waits (weights from HBM, 200 x 2112 x 7168 17.0 ->
+// 13.7 us, 128 x 8192 x 8192 27.3 -> 22.4, 300 x 5000 x 4096 13.4 -> 12.7, 256 x 4096 x 4096
+// 10.9 -> 9.5; row scales: no gain).
 template <bool BLK, class F>
 tb_status with_tile(plan::Fp8Tile tile, int64_t M, int64_t N, const F& f) {
   auto tiles = [&](int64_t tm, int64_t tn) { return (M + tm - 1) / tm * ((N + tn - 1) / tn); };

@@ -21,8 +21,9 @@
 // four consecutive output columns per accumulator group and stores them
 // straight from registers.  One 256 x 256 tile per block on eight wavefronts
 // (128 x 64 each); grids of too few such tiles run 64 x 64, 64 x 128 or 128 x 128
-// tiles on four (plan::pick_nt_tile).  matmul_int8 at M = N = 2048 (64 tiles of 256 x 256) splits
-// K instead when K is deep: 128 x 128 int8 tiles need 32 KiB of operands per
+// tiles on four (plan::pick_nt_tile).  matmul_int8 on fewer than 256 such tiles splits
+// K instead when K is deep (int8_splits, before a small tile is considered): at M = N =
+// 2048 (64 tiles of 256 x 256) 128 x 128 int8 tiles need 32 KiB of operands per
 // CU per 128-byte K step, about the L2-to-CU bandwidth at the MFMA rate, where
 // 256 x 256 tiles need half that per MAC; each split writes an int32 partial
 // plane and a pass adds the planes (exact, so the split does not change a bit).
@@ -379,7 +380,9 @@ struct Small {
   static constexpr int LDS_BYTES = ST * STAGE > TM * CS ? ST * STAGE : TM * CS;
 };
 
-// An overload of nt_gemm: wave tiles of WM = 32 FI rows, ST stages.
+// An overload of nt_gemm, the name under which the launch manifest and its checks
+// know a plain product: tile rows, tile columns and wave rows (WM = 32 FI) as there,
+// then the ring's stages (2 - 4) where the 256 x 256 kernel has its wave columns (64).
 template <int KIND, int OUT, int TM, int TN, int WM, int ST>
 __global__ void __launch_bounds__(256, 1)
     nt_gemm(const uint8_t* __restrict__ A, const uint8_t* __restrict__ BT, uint8_t* __restrict__ Y, int M, int N,

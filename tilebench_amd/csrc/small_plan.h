@@ -190,7 +190,7 @@ struct DecodePlan {
 // A split grid never has more blocks than CUs, counted as they are launched: pairs of
 // 128-column slabs go to the 8 XCDs in turn, and a block fills a CU, so a pair too many on
 // one XCD would start its blocks a whole block's time later (9 x 6528, K 9920, five splits
-// of 51 slabs, 34 blocks on an XCD of 32 CUs: 19.6 us; 256-column slabs 16.1, now 14.0).
+// of 51 slabs, 34 blocks on an XCD of 32 CUs: 19.6 us; 256-column slabs 16.1, bounded 14.2).
 inline int64_t decode_grid(int cols, int64_t slabs, int splits) {
   return cols == 128 ? ((slabs + 1) / 2 * splits + 7) / 8 * 16 : slabs * splits;
 }

@@ -104,9 +104,9 @@ struct Tile {
 // them, as the reference dequantisation does); the difference stays far below
 // the 1e-2 tolerance.  The eight wave partials are summed in LDS in a fixed
 // order, so results are reproducible bit for bit.
-// Measured at M = 16, us, 256-column slabs alone -> now: K 4096, N 4096 14.4 ->
-// 7.8; K 4096, N 11008 12.8 -> 11.8; K 11008, N 4096 16.0 -> 12.1; K 1024, N 12288
-// 10.1 -> 6.1; K 8192, N 28672 (256 columns) 32.6, 3.6 TB/s.
+// Measured at M = 16 on weights that rotate through HBM, us, 256-column slabs alone ->
+// now: K 4096, N 4096 13.9 -> 8.0; K 4096, N 11008 12.5 -> 11.9; K 11008, N 4096 15.6 ->
+// 11.6; K 1024, N 12288 9.4 -> 5.9; K 8192, N 28672 (256 columns) 32.2, 3.7 TB/s.
 // Across the S blocks of a slab the reduction is a serial split-K: each block
 // writes its fp32 partial through to the device-coherent level, then bumps the
 // slab's arrival counter; the block that arrives last reads the S partials
