@@ -515,3 +515,23 @@ def test_fp8_block_scales_at_the_largest_k(gpu, M, N, tile):
     # 128-term and 512-term fp32 sums: (128 + 512) roundings of 2^-24 of the sum of magnitudes at most
     bound = 2.0 ** -8 * want.abs() + 640 * 2.0 ** -24 * size
     assert bool(((Y[r, c].double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dt,op", [("fp16", "OP_MATMUL_F16"), ("fp32", "OP_MATMUL_F32"), ("fp8", "OP_MATMUL_FP8")])
+def test_plain_product_rows_do_not_depend_on_the_tile(gpu, dt, op):
+    """The first M rows alone give the bits they have in a product of 256 x 256 tiles."""
+    from tilebench_amd.benchmarks.operators.matmul_fp32_fp16_fp8 import impl_hip
+
+    N, K, tdt = {"fp16": (4104, 576, torch.float16), "fp32": (4104, 384, torch.float32),
+                 "fp8": (4104, 1152, torch.float8_e4m3fn)}[dt]
+    tile = lambda m: tuple(rt.gemm_tile(getattr(rt, op), m, N, K)[k] for k in ("BM", "BN"))
+    a, b = (t.to(gpu) for t in T.generate_matmul_fp32_fp16_fp8_inputs(4096, N, K, dtype=tdt, seed=5, device="cpu"))
+    big, seen = impl_hip.run(a, b), set()
+    assert tile(4096) == (256, 256)
+    for M in (100, 400, 1000):
+        _say("plain rows", dt, M, N, K, tile(M))
+        seen.add(tile(M))
+        small = impl_hip.run(a[:M].contiguous(), b)
+        torch.cuda.synchronize()
+        assert torch.equal(small.view(torch.uint8), big[:M].contiguous().view(torch.uint8))
+    assert seen == {(64, 64), (64, 128), (128, 128)}
